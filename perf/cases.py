@@ -30,6 +30,8 @@ SHAPES = {
 # router logit biases under which top-2 of eight gives expert loads that follow Zipf(1): what a prompt of one topic does
 ZIPF_BIAS = (0.0, -1.158, -1.581, -1.845, -2.033, -2.186, -2.299, -2.398)
 
+RMS_EPS = 1e-5
+
 # projections of the Mixtral shape: q / o, the grouped k / v, the output head
 LINEARS = ((4096, 4096), (1024, 4096), (32000, 4096))
 
@@ -102,24 +104,39 @@ def _vector(gen, shape, std=0.02, mean=0.0):
     return (mean + std * torch.randn(shape, generator=gen, device="cuda")).cpu().numpy()
 
 
+def _weights(gen, case):
+    """One layer's weights on the host: matrices as quantised bytes, vectors as f32."""
+    s = SHAPES[case["shape"]]
+    H, F, E, Fs = s["hidden"], s["ffn"], s["experts"], s["shared"]
+    dt, down = case["dtype"], case["down"]
+    w = {}
+    if Fs:
+        w.update(shared_w1=_blocks(gen, dt, Fs, H), shared_w3=_blocks(gen, dt, Fs, H), shared_w2=_blocks(gen, down, H, Fs),
+                 shared_gate=_vector(gen, (H,)))
+    if case["skewed"]:
+        w.update(gate_bias=np.array(ZIPF_BIAS, dtype=np.float32))
+    if case["kind"] == "stack":
+        w.update(rms_alpha=_vector(gen, (H,), 0.1, 1.0))
+    w.update(w1=[_blocks(gen, dt, F, H) for _ in range(E)])
+    w.update(w3=[_blocks(gen, dt, F, H) for _ in range(E)])
+    w.update(w2=[_blocks(gen, down, H, F) for _ in range(E)])
+    w.update(gate=_vector(gen, (E, H)))
+    return w
+
+
 def _layer(gen, case):
     s = SHAPES[case["shape"]]
-    H, F, E = s["hidden"], s["ffn"], s["experts"]
-    dt, down = case["dtype"], case["down"]
+    w = _weights(gen, case)
     kw = {}
     if s["shared"]:
-        Fs = s["shared"]
-        kw.update(shared_ffn=Fs, shared_w1=_blocks(gen, dt, Fs, H), shared_w3=_blocks(gen, dt, Fs, H), shared_w2=_blocks(gen, down, H, Fs),
-                  shared_gate=_vector(gen, (H,)))
+        kw.update(shared_ffn=s["shared"], shared_w1=w["shared_w1"], shared_w3=w["shared_w3"], shared_w2=w["shared_w2"],
+                  shared_gate=w["shared_gate"])
     if case["skewed"]:
-        kw.update(gate_bias=np.array(ZIPF_BIAS, dtype=np.float32))
+        kw.update(gate_bias=w["gate_bias"])
     if case["kind"] == "stack":
-        kw.update(rms_alpha=_vector(gen, (H,), 0.1, 1.0), rms_eps=1e-5)
-    w1 = [_blocks(gen, dt, F, H) for _ in range(E)]
-    w3 = [_blocks(gen, dt, F, H) for _ in range(E)]
-    w2 = [_blocks(gen, down, H, F) for _ in range(E)]
-    return candle_amd.SparseMoeBlock(H, F, E, s["top_k"], DTYPES[dt][0], _vector(gen, (E, H)), w1, w3, w2,
-                                     ggml_dtype_down=DTYPES[down][0], **kw)
+        kw.update(rms_alpha=w["rms_alpha"], rms_eps=RMS_EPS)
+    return candle_amd.SparseMoeBlock(s["hidden"], s["ffn"], s["experts"], s["top_k"], DTYPES[case["dtype"]][0], w["gate"], w["w1"], w["w3"],
+                                     w["w2"], ggml_dtype_down=DTYPES[case["down"]][0], **kw)
 
 
 def prepare(case, seed):
@@ -174,3 +191,100 @@ def tolerance(case):
         return {"rel": widen * (1.2e-3 if case["tokens"] < 32 else 4.5e-4), "max": widen * 1.4e-2}
     # The next layer quantises that difference again: four layers summed in another order differ by 5.8e-3 and 3.1e-2.
     return {"rel": 2.4e-2, "max": 1.3e-1}
+
+
+# What `run` returns, in 64 bits: the blocks decoded, activations quantised to 8 bits as the quantised products of GGML do
+# (that is part of the result, not an approximation of it), everything else in double precision.
+def _f16(b):
+    return b.contiguous().view(torch.float16).double()
+
+
+def _k_scales(b):
+    """The eight 6-bit scales and minimums of Q4_K and Q5_K blocks, from their twelve bytes."""
+    b = b.int()
+    lo, mid, hi = b[:, 0:4], b[:, 4:8], b[:, 8:12]
+    return torch.cat((lo & 63, (hi & 15) | (lo >> 6 << 4)), 1).double(), torch.cat((mid & 63, (hi >> 4) | (mid >> 6 << 4)), 1).double()
+
+
+def _decode(dtype, raw, rows, cols):
+    _, _, size = DTYPES[dtype]
+    b = torch.from_numpy(np.ascontiguousarray(raw).view(np.uint8).reshape(-1, size)).cuda()
+    if dtype == "q8_0":
+        x = _f16(b[:, :2]) * b[:, 2:].view(torch.int8).double()
+    elif dtype == "q4_0":
+        q = b[:, 2:]
+        x = _f16(b[:, :2]) * (torch.cat((q & 15, q >> 4), 1).double() - 8)
+    elif dtype == "q6_k":
+        lo, hi, sc = b[:, :128].reshape(-1, 2, 2, 32), b[:, 128:192].reshape(-1, 2, 1, 32), b[:, 192:208].view(torch.int8).double()
+        q = torch.cat((lo & 15, lo >> 4), 2) | (torch.cat([hi >> s & 3 for s in (0, 2, 4, 6)], 2) << 4)
+        x = ((q.reshape(-1, 16, 16).double() - 32) * sc[:, :, None]).reshape(-1, 256) * _f16(b[:, 208:210])
+    else:
+        sc, mn = _k_scales(b[:, 4:16])
+        q = b[:, size - 128:].reshape(-1, 4, 1, 32)
+        q = torch.cat((q & 15, q >> 4), 2).reshape(-1, 8, 32)
+        if dtype == "q5_k":
+            q = q | (torch.stack([b[:, 16:48] >> s & 1 for s in range(8)], 1) << 4)
+        x = (_f16(b[:, :2]) * sc)[:, :, None] * q.double() - (_f16(b[:, 2:4]) * mn)[:, :, None]
+    return x.reshape(rows, cols)
+
+
+def _quantised(dtype, x):
+    """The rows as the quantised product sees them: blocks of 256 (Q8_K) beside K-quants, of 32 (Q8_0) beside the others."""
+    n = DTYPES[dtype][1]
+    v = x.float().reshape(-1, n)
+    amax, at = v.abs().max(1, keepdim=True)
+    if n == 256:
+        inv = -128.0 / v.gather(1, at)
+        d = 1.0 / inv
+    else:
+        d = amax / 127.0
+        inv = 1.0 / d
+        d = d.half()
+    t = (v * inv).double()
+    q = torch.sign(t) * torch.floor(t.abs() + 0.5)
+    return torch.where(amax > 0, q.clamp(-128, 127) * d.double(), 0.0).reshape(x.shape)
+
+
+def _expert(case, x, ffn, w1, w3, w2):
+    H = x.shape[1]
+    xq = _quantised(case["dtype"], x)
+    a, b = xq @ _decode(case["dtype"], w1, ffn, H).T, xq @ _decode(case["dtype"], w3, ffn, H).T
+    h = a * torch.sigmoid(a) * b
+    # One layer: the intermediate stays in 64 bits.  Rounded to 8 bits as the layer does, its last bits decide which step a
+    # value takes, and an equally good sum in another order is 1e-7 off by luck or 1e-4.  In a stack the steps of the layers
+    # before are part of what a layer reads.
+    return (_quantised(case["down"], h) if case["kind"] == "stack" else h) @ _decode(case["down"], w2, H, ffn).T
+
+
+def _block64(case, w, x):
+    s = SHAPES[case["shape"]]
+    vec = lambda name: torch.from_numpy(w[name]).cuda().double()
+    xs = x
+    if "rms_alpha" in w:
+        xs = (x / (x.square().mean(1, keepdim=True) + RMS_EPS).sqrt() * vec("rms_alpha")).float().double()   # an f32 row in the model
+    probs = torch.softmax(xs @ vec("gate").T + (vec("gate_bias") if "gate_bias" in w else 0.0), 1)
+    top, idx = probs.topk(s["top_k"], 1)
+    top = top / top.sum(1, keepdim=True)
+    y = x.clone() if "rms_alpha" in w else torch.zeros_like(x)
+    for e in range(s["experts"]):
+        t, r = (idx == e).nonzero(as_tuple=True)
+        if len(t):
+            y.index_add_(0, t, top[t, r, None] * _expert(case, xs[t], s["ffn"], w["w1"][e], w["w3"][e], w["w2"][e]))
+    if s["shared"]:
+        y += torch.sigmoid(xs @ vec("shared_gate"))[:, None] * _expert(case, xs, s["shared"], w["shared_w1"], w["shared_w3"], w["shared_w2"])
+    return y
+
+
+def exact(case, seed):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    T = case["tokens"]
+    if case["kind"] == "linear":
+        n, k = case["n"], case["k"]
+        w = _decode(case["dtype"], _blocks(gen, case["dtype"], n, k), n, k)
+        return _quantised(case["dtype"], torch.randn((T, k), generator=gen, device="cuda")) @ w.T
+    layers = [_weights(gen, case) for _ in range(case["layers"])]
+    x = torch.randn((T, SHAPES[case["shape"]]["hidden"]), generator=gen, device="cuda").double()
+    for w in layers:
+        x = _block64(case, w, x)
+    return x.cpu().numpy() if case["kind"] == "host" else x
