@@ -82,7 +82,7 @@ def build_library(verbose=False, out_dir=None, extra_flags=()):
 if __name__ == "__main__":
     import argparse
     ap = argparse.ArgumentParser(description="Builds libcandle_amd_moe.so; --out-dir / --flag: a second library beside the "
-                                             "product's (measurement variants such as -DMOE_WHATIF=N of kernels_q4k_gemm.hip)")
+                                             "product's")
     ap.add_argument("--out-dir", default=None)
     ap.add_argument("--flag", action="append", default=[])
     a = ap.parse_args()

@@ -10,15 +10,22 @@
 // the whole 256-element super-block.  8*acc_hi + acc_lo is then the exact integer the reference
 // computes; the mins term is an exact f16 MFMA over the 16 block sums.
 //
-// Work split: a workgroup (8 waves) owns one tile of 128 slots of one expert (from the dispatch
-// kernel's tile list, so a skewed routing is balanced by tiles, not by experts) and eight 16-row
-// weight operands, one per wave.  The 128 activation rows of a super-block go straight from global
+// Work split: a workgroup (8 or 4 waves) owns one tile of 128 or 64 slots of one expert (from the dispatch
+// kernel's tile list, so a skewed routing is balanced by tiles, not by experts) and two 16-row
+// weight operands per wave.  The activation rows of a super-block go straight from global
 // memory into LDS (double-buffered, no staging registers) and every wave reads them as MFMA A
-// operands.  A wave unpacks and pre-scales its 16 weight rows of the super-block once, keeps the two
-// planes in registers (32 VGPRs) and runs them against the eight 16-slot operands one after the other.
-// The 16-row operand keeps a wave below 128 VGPRs, so four waves share a SIMD: a single wave issues
-// at most one vector instruction every ~5 cycles and stalls on every MFMA result, and it takes that
-// many waves to keep the MFMA pipe and the vector ALU busy at the same time.
+// operands.  A wave unpacks and pre-scales its 32 weight rows of the super-block once, keeps the
+// planes in registers (64 VGPRs) and runs them against the 16-slot operands one after the other.
+//
+// What bounds it: the issue port of a SIMD, which matrix and vector instructions share (a 16x16x64 MFMA holds it for 8
+// cycles, a vector instruction for 4), with the unpacking (95 vector instructions per 16 rows and super-block) and the
+// results (5 each).  Two weight operands per wave: an LDS read feeds four matrix instructions instead of two.  That
+// takes two waves per SIMD (256 registers), too few to cover each other, so a wave overlaps its own work: the results of
+// operand o - 1 are added up between the matrix instructions of operand o, and the next super-block's transfers are
+// issued a few at a time behind the operands (in one go at the top they held each wave up for 1650 to 4700 of 9000 cycles).
+// Up launch, 4096 tokens at the Mixtral shape: one operand per wave, four waves per SIMD 2.26 ms, this kernel 1.97 ms;
+// the same with 32x32x32 MFMAs and no overlap in the wave 2.3 ms.  Operands beyond a short tile's list are neither
+// fetched nor multiplied (the K loop exists for 8, 6, 4 and 2 of them).
 //
 // Q6K weights (the w2 of mixed files) take the same kernel for the down projection.  BlockQ6K::vec_dot
 // (k_quants.rs:1613-1671) is d * y.d * sum_j sc_j * ((code_j - 32) . q8_j) with an i8 scale per 16 elements; the
@@ -32,6 +39,7 @@
 #include <type_traits>
 #include "act_quant.hpp"
 #include "kernels.hpp"
+#include "planes.hpp"
 
 namespace moe {
 
@@ -49,7 +57,6 @@ __device__ __forceinline__ T gld(const void* uniform_base, uint32_t off) {
 
 // four bytes (each <= 15) times a digit (<= 7): no byte overflows, and the packed 16-bit multiply does
 // both halves of the register in one full-rate instruction (a 24-bit multiply would drop the top byte)
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t scale_bytes(uint32_t q, uint32_t s) {
     const u16x2 a = __builtin_bit_cast(u16x2, q);
     const u16x2 b = {(unsigned short)s, (unsigned short)s};
@@ -90,38 +97,38 @@ __device__ __forceinline__ void dma4(const void* gbase, uint32_t voff, uint32_t 
 }
 __device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0)
 
-// Measurement aid, Q4K only, never set in the product (`python -m candle_amd.build --out-dir DIR --flag=-DMOE_WHATIF=N`
-// builds a second library; its results are WRONG by construction, only its kernel times mean something).  Each bit
-// takes one cost out of the tiled kernel's K loop, to show what the loop's other parts alone would take:
-//   1  the result step: one vector instruction per result keeps the matrix instructions alive, no mins product
-//   2  the unpacking of the weights into two scaled digit planes (the raw bytes go to the matrix cores)
-//   4  the transfers of the next super-block's activations into LDS
-//   8  the LDS reads of the activation operands (one register set for every operand)
-#ifndef MOE_WHATIF
-#define MOE_WHATIF 0
-#endif
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(const F& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
 
 // What a lane fetches for the tile.  Quants: the NOP*4 (operand, pair) stretches of 1 KiB are dealt to
-// the eight waves, NOP/2 each: lane (m = l%16, g = l/16) fetches piece (P, g) of row 16 o + m.  Block
+// the NW waves, NB each: lane (m = l%16, g = l/16) fetches piece (P, g) of row 16 o + m.  Block
 // sums: one transfer covers two operands: lane fetches half (l/16)%2 of row 32 x + 16 (l/32) + l%16.
 // Scales: row 64 x + l.  Waves without a share of the sums and scales repeat another wave's transfer:
 // same bytes to the same place, and no branch around a load.
+template <int NB>
 struct StageRows {
-    uint32_t q;        // byte offset of the row's quants
-    uint32_t bs, yd;   // row index
+    // byte offsets of the lane's first-super-block bytes; a transfer's super-block and pair are in its (scalar) base address
+    uint32_t q[(NB + 3) / 4];   // per operand of the wave's share
+    uint32_t bs, yd;
 };
-// transfer number I (0 .. NOP/2+1) of a wave's share of the tile: NOP/2 quant stretches, block sums, scales
-template <int I, int NOP>
-__device__ __forceinline__ void stage_piece(const ActBuf& ab, const StageRows& r, int nsb, int sb, GemmLds<NOP>& L, int buf, int wave, int lane) {
-    constexpr int NB = NOP / 2;
-    if (I < NB) {
-        const int blk = wave * NB + I;            // = 4 o + P with o the wave's operand (r.q is its row)
-        dma16(ab.qs, r.q + (uint32_t)(sb * 256 + ((blk & 3) * 4 + (lane >> 4)) * 16), lds_address(L.q[buf]) + (uint32_t)(blk * 1024));
-    } else if (I == NB) {
-        dma16(ab.bsum, ((r.bs * (uint32_t)nsb + (uint32_t)sb) * 16 + ((lane >> 4) & 1) * 8) * 2,
-              lds_address(&L.bs[buf][0][0][0][0]) + (uint32_t)((wave % (NOP / 2)) * 1024));
+// transfer number I of a wave's share: quant stretches 0 .. NB-1, then the block sums, then the scales
+template <int I, bool SUMS, int NOP, int NB>
+__device__ __forceinline__ void stage_piece(const ActBuf& ab, const StageRows<NB>& r, int sb, GemmLds<NOP>& L, int buf, int wave, int live) {
+    if constexpr (I < NB) {
+        const int blk = wave * NB + I;      // = 4 o + P
+        if ((blk >> 2) < live)              // (operands beyond the list are never read)
+            dma16(ab.qs + sb * 256 + (blk & 3) * 64, r.q[I / 4], lds_address(L.q[buf]) + (uint32_t)(blk * 1024));
+    } else if constexpr (I == NB) {
+        if constexpr (SUMS)
+            dma16(static_cast<const uint8_t*>(ab.bsum) + sb * 32, r.bs,
+                  lds_address(&L.bs[buf][0][0][0][0]) + (uint32_t)((wave % (NOP / 2)) * 1024));
     } else {
-        dma4(ab.d, (r.yd * (uint32_t)nsb + (uint32_t)sb) * 4, lds_address(&L.yd[buf][0]) + (uint32_t)((wave % (NOP / 4)) * 256));
+        dma4(ab.d + sb, r.yd, lds_address(&L.yd[buf][0]) + (uint32_t)((wave % (NOP / 4)) * 256));
     }
 }
 
@@ -174,18 +181,6 @@ struct BPlanes {
 __device__ __forceinline__ BPlanes b_prepare(const BRegs& b, int lane) {
     const int g = lane >> 4;
     const uint32_t M4 = 0x0f0f0f0fu;
-    if (MOE_WHATIF & 2) {   // measurement aid: no unpacking
-        BPlanes o;
-        o.d = __uint_as_float(b.hdr.x); o.dmin = __uint_as_float(b.hdr.y);
-#pragma unroll
-        for (int P = 0; P < 4; P++) {
-            const u32x4 c = b.c[P >> 1];
-            o.lo[P] = v4i{(int)c.x, (int)c.y, (int)c.z, (int)c.w};
-            o.hi[P] = v4i{(int)c.y, (int)c.z, (int)c.w, (int)c.x};
-        }
-        o.mB = v4h{0, 0, 0, 0};
-        return o;
-    }
     const uint32_t u0 = b.hdr.y, u1 = b.hdr.z, u2 = b.hdr.w;
     BPlanes o;
     o.d = __half2float(__ushort_as_half((unsigned short)(b.hdr.x & 0xffffu)));
@@ -215,20 +210,7 @@ __device__ __forceinline__ BPlanes b_prepare(const BRegs& b, int lane) {
     return o;
 }
 
-// Q6K: both planes of W = sc * (code - 32).  A word of four codes is spread over two registers of two 16-bit lanes
-// (even and odd bytes), each multiplied and offset in one packed multiply-add: W + 128 = code * sc + (128 - 32 sc).
-// The high bytes of W + 128 are H = floor((W + 128) / 256); its low bytes, with the top bit flipped, are W - 256 H as a
-// signed byte.
-__device__ __forceinline__ uint32_t pk_mad_u16(uint32_t a, uint32_t b, uint32_t c) {
-    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) + __builtin_bit_cast(u16x2, c)));
-}
-__device__ __forceinline__ void q6k_planes(uint32_t codes, uint32_t s2, uint32_t add2, int& lo, int& hi) {
-    const uint32_t ev = codes & 0x00ff00ffu;
-    const uint32_t od = __builtin_amdgcn_perm(0u, codes, 0x0c030c01u);
-    const uint32_t we = pk_mad_u16(ev, s2, add2), wo = pk_mad_u16(od, s2, add2);
-    lo = (int)(__builtin_amdgcn_perm(wo, we, 0x06020400u) ^ 0x80808080u);
-    hi = (int)__builtin_amdgcn_perm(wo, we, 0x07030501u);
-}
+// Q6K: both planes of W = sc * (code - 32) (planes.hpp).
 __device__ __forceinline__ BPlanes b_prepare_q6k(const BRegs& b, int lane) {
     const int g = lane >> 4;
     const uint32_t M4 = 0x0f0f0f0fu, M2H = 0x30303030u;
@@ -352,76 +334,105 @@ __device__ __forceinline__ BPlanes b_prepare_q2k(const BRegs& b, int lane) {
     return o;
 }
 
-// one super-block of the wave's 16 weight rows against 16-slot operand o of the staged tile
-// `while_busy` runs right after the MFMAs are issued: this is where the next super-block's loads go.
-template <int FMT, int NOP, typename Fill>
-__device__ __forceinline__ void gemm_operand(const BPlanes& B, const GemmLds<NOP>& L, int buf, int o, int lane, v4f& facc, Fill while_busy) {
+template <int FMT>
+__device__ __forceinline__ BPlanes b_planes(const BRegs& r, int lane) {
+    if constexpr (FMT == MOE_GGML_Q6K) return b_prepare_q6k(r, lane);
+    else if constexpr (FMT == MOE_GGML_Q2K) return b_prepare_q2k(r, lane);
+    else if constexpr (FMT == MOE_GGML_Q3K) return b_prepare_q3k(r, lane);
+    else if constexpr (FMT == MOE_GGML_Q5K) return b_prepare_q5k(r, lane);
+    else return b_prepare(r, lane);
+}
+
+// The matrix results of one 16-slot operand against the wave's two 16-row weight operands, on their way to the sums.
+struct OperandAcc {
+    v4i lo[2], hi[2];
+    v4f dm[2], yd;
+};
+// Adds result i (slot 16 o + 4 g + i, weight rows n = lane%16 of both operands) of a super-block to the sums.
+template <int FMT>
+__device__ __forceinline__ void gemm_result(const BPlanes (&B)[2], const OperandAcc& A, int i, v4f (&facc)[2]) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if constexpr (FMT == MOE_GGML_Q6K || FMT == MOE_GGML_Q3K) {
+            const int isum = (A.hi[j][i] << 8) + A.lo[j][i];
+            facc[j][i] = __builtin_fmaf(B[j].d * A.yd[i], (float)isum, facc[j][i]);
+        } else if constexpr (FMT == MOE_GGML_Q2K) {
+            // the reference's own order, every product and the difference rounded (k_quants.rs:772-773, 801): with unsigned
+            // 2-bit codes the two terms are large and nearly cancel, and the scalar path's sum has one order only -- a
+            // wave walks K in that order, so the up projection repeats vec_dot_unopt bit for bit
+            const float dall = A.yd[i] * B[j].d, dminy = A.yd[i] * B[j].dmin;
+            facc[j][i] += dall * (float)A.lo[j][i] - dminy * A.dm[j][i];
+        } else {
+            const int isum = (A.hi[j][i] << (FMT == MOE_GGML_Q5K ? 8 : 3)) + A.lo[j][i];
+            const float v = __builtin_fmaf(B[j].d, (float)isum, -(B[j].dmin * A.dm[j][i]));
+            facc[j][i] = __builtin_fmaf(A.yd[i], v, facc[j][i]);
+        }
+        float f = facc[j][i];
+        asm volatile("" : "+v"(f));   // the step stays where it is written
+        facc[j][i] = f;
+    }
+}
+__device__ __forceinline__ v4i operand_piece(const uint8_t* q, int o, int P, int lane) {
+    return *reinterpret_cast<const v4i*>(q + o * 4096 + P * 1024 + lane * 16);
+}
+// One super-block of the wave's 32 weight rows against operands O, O + 1, ... of the staged tile.  While the matrix
+// instructions of an operand run, the wave's vector instructions add up the results of the operand before it (`prev`).
+template <int FMT, int NOP, int LV, int O, class Fill>
+__device__ __forceinline__ void gemm_operands(const BPlanes (&B)[2], const GemmLds<NOP>& L, int buf, int lane, v4i (&a)[4], OperandAcc& prev,
+                                              v4f (&facc)[NOP][2], const Fill& fill) {
     const int m = lane & 15, g = lane >> 4;
     const v4i zero4 = {0, 0, 0, 0};
-    v4i acc_lo, acc_hi;
-    const uint8_t* arow = L.q[buf] + o * 4096 + lane * 16;
-    // the wave takes issue priority while its matrix instructions go out: they keep the matrix pipe fed while the other
-    // waves of the SIMD work through their result steps (2 % on the kernel)
-    __builtin_amdgcn_s_setprio(2);
+    OperandAcc cur;
+    v4h mA;
+    if constexpr (FMT != MOE_GGML_Q6K && FMT != MOE_GGML_Q3K) mA = *reinterpret_cast<const v4h*>(&L.bs[buf][O][g >> 1][m][(g & 1) * 4]);
+    cur.yd = *reinterpret_cast<const v4f*>(&L.yd[buf][O * 16 + g * 4]);
 #pragma unroll
     for (int P = 0; P < 4; P++) {
-        v4i a;
-        if (MOE_WHATIF & 8) a = v4i{lane, lane + 1, lane + 2, lane + 3};   // measurement aid: no LDS read (one register set for all)
-        else a = *reinterpret_cast<const v4i*>(arow + P * 1024);
-        acc_lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, B.lo[P], P == 0 ? zero4 : acc_lo, 0, 0, 0);
-        if constexpr (FMT != MOE_GGML_Q2K) acc_hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, B.hi[P], P == 0 ? zero4 : acc_hi, 0, 0, 0);
-    }
-    __builtin_amdgcn_s_setprio(0);
-    // D[i] belongs to slot 16 o + 4 g + i, weight row n = lane%16
-    if constexpr (FMT == MOE_GGML_Q6K || FMT == MOE_GGML_Q3K) {
-        const v4f yd = *reinterpret_cast<const v4f*>(&L.yd[buf][o * 16 + g * 4]);
-        while_busy();
+        const v4i x = a[P];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int isum = (acc_hi[i] << 8) + acc_lo[i];
-            facc[i] = __builtin_fmaf(B.d * yd[i], (float)isum, facc[i]);
+        for (int j = 0; j < 2; j++) {
+            cur.lo[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, B[j].lo[P], P == 0 ? zero4 : cur.lo[j], 0, 0, 0);
+            if constexpr (FMT != MOE_GGML_Q2K) cur.hi[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, B[j].hi[P], P == 0 ? zero4 : cur.hi[j], 0, 0, 0);
         }
-    } else if ((MOE_WHATIF & 1) && FMT == MOE_GGML_Q4K) {   // measurement aid: no result step
-        while_busy();
-#pragma unroll
-        for (int i = 0; i < 4; i++) facc[i] = __int_as_float(acc_lo[i] + acc_hi[i] + __float_as_int(facc[i]));
-    } else {
-        const v4h mA = *reinterpret_cast<const v4h*>(&L.bs[buf][o][g >> 1][m][(g & 1) * 4]);
+        if constexpr (O + 1 < LV) a[P] = operand_piece(L.q[buf], O + 1, P, lane);
+        if constexpr (O > 0) gemm_result<FMT>(B, prev, P, facc[O - 1]);
+        // order: a matrix instruction (mask 0x8), three vector instructions (0x2), and so on
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 9, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (P == 0) fill(std::integral_constant<int, O>{});
+    }
+    if constexpr (FMT != MOE_GGML_Q6K && FMT != MOE_GGML_Q3K) {
         const v4f zf = {0.f, 0.f, 0.f, 0.f};
-        const v4f Dm = __builtin_amdgcn_mfma_f32_16x16x16f16(mA, B.mB, zf, 0, 0, 0);
-        const v4f yd = *reinterpret_cast<const v4f*>(&L.yd[buf][o * 16 + g * 4]);
-        while_busy();
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            if constexpr (FMT == MOE_GGML_Q2K) {
-                // the reference's own order, every product and the difference rounded (k_quants.rs:772-773, 801): with unsigned
-                // 2-bit codes the two terms are large and nearly cancel, and the scalar path's sum has one order only -- a
-                // wave walks K in that order, so the up projection repeats vec_dot_unopt bit for bit
-                const float dall = yd[i] * B.d, dminy = yd[i] * B.dmin;
-                facc[i] += dall * (float)acc_lo[i] - dminy * Dm[i];
-            } else {
-                const int isum = (acc_hi[i] << (FMT == MOE_GGML_Q5K ? 8 : 3)) + acc_lo[i];
-                const float v = __builtin_fmaf(B.d, (float)isum, -(B.dmin * Dm[i]));
-                facc[i] = __builtin_fmaf(yd[i], v, facc[i]);
-            }
-        }
+        for (int j = 0; j < 2; j++) cur.dm[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(mA, B[j].mB, zf, 0, 0, 0);
     }
+    prev = cur;
+    if constexpr (O + 1 < LV) {
+        gemm_operands<FMT, NOP, LV, O + 1>(B, L, buf, lane, a, prev, facc, fill);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) gemm_result<FMT>(B, prev, i, facc[O]);
 }
 
 __device__ __forceinline__ float silu_gemm(float v) { return v / (1.0f + __expf(-v)); }
 
 // ---------------------------------------------------------------------------------------------
-// One 16-row weight operand per wave, eight waves per workgroup, two workgroups per CU; a tile of
-// NOP*16 slots.
-// MODE 0: up   -- a workgroup owns 64 rows of F: waves 0-3 carry those rows of w1, waves 4-7 the same
-//                 rows of w3; the w3 waves hand their sums over through LDS and the w1 waves write
-//                 h = silu(a) * b (f32).
-// MODE 1: down -- a workgroup owns 128 rows of H of w2, one 16-row operand per wave; writes yw.
+// Two 16-row weight operands per wave, NW waves per workgroup, two waves per SIMD; a tile of NOP*16 slots.
+// MODE 0: up   -- a wave carries 16 rows of w1 and the same 16 rows of w3 and writes h = silu(a) * b (f32).
+// MODE 1: down -- 32 rows of w2 per wave; writes yw.
 // FMT: the weights' format (Q2K ... Q6K).
-template <int FMT, int MODE, int NOP>
-__global__ __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void q4k_gemm_kernel(ExpertParams p) {
+template <int FMT, int MODE, int NOP, int NW>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void q4k_gemm_kernel(ExpertParams p) {
     static_assert(FMT == MOE_GGML_Q2K || FMT == MOE_GGML_Q3K || FMT == MOE_GGML_Q4K || FMT == MOE_GGML_Q5K || FMT == MOE_GGML_Q6K, "formats of the tiled kernel");
-    constexpr int NB = NOP / 2;
+    constexpr int NB = NOP * 4 / NW;
     constexpr int TILE_BYTES = FMT == MOE_GGML_Q6K ? Q6K_TILE_BYTES : FMT == MOE_GGML_Q5K ? Q5K_TILE_BYTES : FMT == MOE_GGML_Q2K ? Q2K_TILE_BYTES : FMT == MOE_GGML_Q3K ? Q3K_TILE_BYTES : Q4K_TILE_BYTES;
     constexpr bool kSums = FMT != MOE_GGML_Q6K && FMT != MOE_GGML_Q3K;   // block sums staged (the mins term)
     __shared__ GemmLds<NOP> L;
@@ -429,7 +440,7 @@ __global__ __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n_tiles = p.rb.tile_tab[0];
     // workgroup -> (row block, slot tile), in patches per XCD (patch_position)
-    const int n_rb = MODE == 0 ? p.F / 64 : p.H / 128;
+    const int n_rb = MODE == 0 ? p.F / (16 * NW) : p.H / (32 * NW);
     const PatchPos pos = patch_position((int)blockIdx.x, n_rb, p.patch);
     const int rblk = pos.rblk, tile = pos.tile;
     if (tile >= n_tiles || rblk >= n_rb) return;
@@ -449,140 +460,125 @@ __global__ __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)
         const int slot = s_begin + (pos < n_g ? pos : n_g - 1);
         return MODE == 0 ? p.rb.perm_token[slot] : slot - p.slot_origin;
     };
-    StageRows rows;
-    rows.q = (uint32_t)act_row(16 * ((wave * NB) >> 2) + (lane & 15)) * (uint32_t)K;
-    rows.bs = (uint32_t)act_row(32 * (wave % (NOP / 2)) + 16 * (lane >> 5) + (lane & 15));
-    rows.yd = (uint32_t)act_row(64 * (wave % (NOP / 4)) + lane);
-
-    // weight operand of this wave
-    const GroupWeights gw = p.groups[grp];
-    const uint8_t* wp;
-    int row0;
-    if (MODE == 0) {
-        row0 = rblk * 64 + (wave & 3) * 16;
-        wp = (wave < 4 ? gw.w1 : gw.w3) + (size_t)(row0 / 16) * TILE_BYTES;
-    } else {
-        row0 = rblk * 128 + wave * 16;
-        wp = gw.w2 + (size_t)(row0 / 16) * TILE_BYTES;
-    }
-    v4f facc[NOP];
+    StageRows<NB> rows;
 #pragma unroll
-    for (int o = 0; o < NOP; o++) facc[o] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < (NB + 3) / 4; c++) rows.q[c] = (uint32_t)act_row(16 * (((wave * NB) >> 2) + c) + (lane & 15)) * (uint32_t)K + (lane >> 4) * 16;
+    rows.bs = ((uint32_t)act_row(32 * (wave % (NOP / 2)) + 16 * (lane >> 5) + (lane & 15)) * (uint32_t)nsb * 16 + ((lane >> 4) & 1) * 8) * 2;
+    rows.yd = (uint32_t)act_row(64 * (wave % (NOP / 4)) + lane) * (uint32_t)nsb * 4;
 
-    // transfer t of the wave's share (quant stretches, sums, scales), then the weight tile
-    auto stage = [&](auto I, int sb, int buf) {
-        if ((MOE_WHATIF & 4) && sb > 0) return;   // measurement aid: the first super-block's transfers only
-        if constexpr (!kSums && decltype(I)::value == NB) return;
-        stage_piece<decltype(I)::value, NOP>(ab, rows, nsb, sb, L, buf, wave, lane);
-    };
-    auto prepare = [&](const BRegs& r) {
-        if constexpr (FMT == MOE_GGML_Q6K) return b_prepare_q6k(r, lane);
-        else if constexpr (FMT == MOE_GGML_Q2K) return b_prepare_q2k(r, lane);
-        else if constexpr (FMT == MOE_GGML_Q3K) return b_prepare_q3k(r, lane);
-        else if constexpr (FMT == MOE_GGML_Q5K) return b_prepare_q5k(r, lane);
-        else return b_prepare(r, lane);
-    };
-    using std::integral_constant;
-    stage(integral_constant<int, 0>{}, 0, 0);
-    stage(integral_constant<int, 1>{}, 0, 0);
-    stage(integral_constant<int, NB>{}, 0, 0);
-    stage(integral_constant<int, NB + 1>{}, 0, 0);
-    if constexpr (NB == 4) { stage(integral_constant<int, 2>{}, 0, 0); stage(integral_constant<int, 3>{}, 0, 0); }
-    BRegs raw = b_load<FMT>(wp, lane);
+    // weight operands of this wave
+    const GroupWeights gw = p.groups[grp];
+    const int row0 = (rblk * NW + wave) * (MODE == 0 ? 16 : 32);
+    const uint8_t* wp[2];
+    if (MODE == 0) {
+        wp[0] = gw.w1 + (size_t)(row0 / 16) * TILE_BYTES;
+        wp[1] = gw.w3 + (size_t)(row0 / 16) * TILE_BYTES;
+    } else {
+        wp[0] = gw.w2 + (size_t)(row0 / 16) * TILE_BYTES;
+        wp[1] = wp[0] + TILE_BYTES;
+    }
+    v4f facc[NOP][2];
+#pragma unroll
+    for (int o = 0; o < NOP; o++) facc[o][0] = facc[o][1] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    // operands of the tile that hold slots of the list: a short tile's others are neither fetched nor multiplied
+    const int live = __builtin_amdgcn_readfirstlane(min(NOP, (n_g - pos0 + 15) >> 4));
+    auto stage = [&](auto I, int sb, int buf) { stage_piece<decltype(I)::value, kSums, NOP, NB>(ab, rows, sb, L, buf, wave, live); };
+    static_for<0, NB + 2>([&](auto I) { stage(I, 0, 0); });
+    BRegs raw[2] = {b_load<FMT>(wp[0], lane), b_load<FMT>(wp[1], lane)};
     wait_all_loads();
     __syncthreads();
-    for (int sb = 0; sb < nsb; sb++) {
-        const int buf = sb & 1, nb = buf ^ 1;
-        const int sbn = sb + 1 < nsb ? sb + 1 : sb;
-        const BPlanes B = prepare(raw);
-        // the next super-block's activations and weights are requested while the operands' MFMAs drain
-        if constexpr (NOP == 8) {
-            gemm_operand<FMT>(B, L, buf, 0, lane, facc[0], [&] { stage(integral_constant<int, 0>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 1, lane, facc[1], [&] { stage(integral_constant<int, 1>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 2, lane, facc[2], [&] { stage(integral_constant<int, 2>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 3, lane, facc[3], [&] { stage(integral_constant<int, 3>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 4, lane, facc[4], [&] { stage(integral_constant<int, 4>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 5, lane, facc[5], [&] { stage(integral_constant<int, 5>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 6, lane, facc[6], [&] { raw = b_load<FMT>(wp + (size_t)sbn * sb_stride, lane); });
-            gemm_operand<FMT>(B, L, buf, 7, lane, facc[7], [&] {});
-        } else {
-            gemm_operand<FMT>(B, L, buf, 0, lane, facc[0], [&] { stage(integral_constant<int, 0>{}, sbn, nb); stage(integral_constant<int, 1>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 1, lane, facc[1], [&] { stage(integral_constant<int, NB>{}, sbn, nb); stage(integral_constant<int, NB + 1>{}, sbn, nb); });
-            gemm_operand<FMT>(B, L, buf, 2, lane, facc[2], [&] { raw = b_load<FMT>(wp + (size_t)sbn * sb_stride, lane); });
-            gemm_operand<FMT>(B, L, buf, 3, lane, facc[3], [&] {});
+    // the K loop over LV operands
+    auto run = [&](auto lv_tag) {
+        constexpr int LV = decltype(lv_tag)::value;
+        for (int sb = 0; sb < nsb; sb++) {
+            const int buf = sb & 1, nb = buf ^ 1;
+            const int sbn = sb + 1 < nsb ? sb + 1 : sb;
+            const BPlanes B[2] = {b_planes<FMT>(raw[0], lane), b_planes<FMT>(raw[1], lane)};
+            // (for the sake of the registers the next weights are requested after this super-block's are unpacked)
+            __builtin_amdgcn_sched_barrier(0);
+            v4i a[4];
+#pragma unroll
+            for (int P = 0; P < 4; P++) a[P] = operand_piece(L.q[buf], 0, P, lane);
+            OperandAcc prev;
+            // The next super-block's weights and activations are requested while the operands are multiplied, a few requests at a
+            // time: issued in one go they fill the CU's memory queue and the wave stands still for a thousand cycles and more.
+            gemm_operands<FMT, NOP, LV, 0>(B, L, buf, lane, a, prev, facc, [&](auto o_tag) {
+                constexpr int O = decltype(o_tag)::value;
+                if constexpr (O == 0) raw[0] = b_load<FMT>(wp[0] + (size_t)sbn * sb_stride, lane);
+                if constexpr (O == (LV > 2 ? 1 : 0)) raw[1] = b_load<FMT>(wp[1] + (size_t)sbn * sb_stride, lane);
+                constexpr int FIRST = LV > 2 ? 1 : 0, SPAN = LV > 4 ? LV - 3 : 1;
+                static_for<0, NB + 2>([&](auto I) {
+                    if constexpr (FIRST + decltype(I)::value * SPAN / (NB + 2) == O) stage(I, sbn, nb);
+                });
+            });
+            wait_all_loads();
+            __syncthreads();
         }
-        wait_all_loads();
-        __syncthreads();
-    }
+    };
+    if (live > NOP * 3 / 4) run(std::integral_constant<int, NOP>{});
+    else if (live > NOP / 2) run(std::integral_constant<int, NOP * 3 / 4>{});
+    else if (NOP == 4 || live > NOP / 4) run(std::integral_constant<int, NOP / 2>{});
+    else run(std::integral_constant<int, NOP / 4>{});
 
-    // epilogue: lane holds weight row n = lane%16 and slots 16 o + 4 (lane/16) + i
+    // epilogue: lane holds weight row n = lane%16 of both operands and slots 16 o + 4 (lane/16) + i
     const int n = lane & 15, g = lane >> 4;
-    if (MODE == 0) {
-        // w3 waves (4-7) park their sums in LDS (the activation buffers are free now), w1 waves combine
-        float* xch = reinterpret_cast<float*>(L.q[0]);   // [4 waves][NOP][4 i][64 lanes] floats
-        static_assert(4 * NOP * 4 * 64 * 4 <= sizeof(L.q), "exchange area");
-        if (wave >= 4) {
 #pragma unroll
-            for (int o = 0; o < NOP; o++)
+    for (int o = 0; o < NOP; o++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) xch[(((wave - 4) * NOP + o) * 4 + i) * 64 + lane] = facc[o][i];
-        }
-        __syncthreads();
-        if (wave < 4) {
-#pragma unroll
-            for (int o = 0; o < NOP; o++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int pos = pos0 + o * 16 + g * 4 + i;
-                    if (pos >= n_g) continue;
-                    const float bsum = xch[((wave * NOP + o) * 4 + i) * 64 + lane];
-                    p.hbuf[(int64_t)(s_begin + pos - p.slot_origin) * p.F + row0 + n] = silu_gemm(facc[o][i]) * bsum;
-                }
-        }
-    } else {
-#pragma unroll
-        for (int o = 0; o < NOP; o++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int pos = pos0 + o * 16 + g * 4 + i;
-                if (pos >= n_g) continue;
-                const int slot = s_begin + pos;
-                p.yw[(int64_t)slot * p.H + row0 + n] = facc[o][i] * p.rb.perm_w[slot];
+        for (int i = 0; i < 4; i++) {
+            const int pos = pos0 + o * 16 + g * 4 + i;
+            if (pos >= n_g) continue;
+            const int slot = s_begin + pos;
+            if (MODE == 0) {
+                p.hbuf[(int64_t)(slot - p.slot_origin) * p.F + row0 + n] = silu_gemm(facc[o][0][i]) * facc[o][1][i];
+            } else {
+                const float w = p.rb.perm_w[slot];
+                p.yw[(int64_t)slot * p.H + row0 + n] = facc[o][0][i] * w;
+                p.yw[(int64_t)slot * p.H + row0 + 16 + n] = facc[o][1][i] * w;
             }
-    }
+        }
 }
 
 template <int FMT, int MODE>
-static void launch_gemm(const ExpertParams& p, dim3 grid, hipStream_t s) {
-    if (p.rb.tile_slots == 64) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4>), grid, dim3(G_THREADS), 0, s, p);
-    else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8>), grid, dim3(G_THREADS), 0, s, p);
+static void launch_gemm(ExpertParams& p, hipStream_t s) {
+    const int64_t tiles = max_gemm_tiles(p.n_slots, p.n_groups + 1, p.rb.tile_slots);
+    const int64_t rows = MODE == 0 ? 2 * (int64_t)p.F : p.H;
+    // Workgroups of eight waves (256 weight rows) fetch an activation tile half as often as those of four.  (Mixtral shape, Q4_K,
+    // us, eight / four waves: 301 tokens 467 / 519, 4096 tokens 3210 / 3282; 777 rows x 4096 x 4096, 208 / 416 workgroups of
+    // 64 slots: 54 / 58.)  A grid that would leave half of the CUs without one takes the four-wave ones.
+    const bool wide = rows % 256 == 0 && rows / 256 * tiles >= 128;
+    const int64_t n_rb = rows / (wide ? 256 : 128);
+    p.patch = patch_edge(n_rb, tiles);
+    const dim3 grid(patch_grid(n_rb, tiles, p.patch));
+    if (p.rb.tile_slots == 64) {
+        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8>), grid, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4>), grid, dim3(256), 0, s, p);
+    } else {
+        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 8>), grid, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 4>), grid, dim3(256), 0, s, p);
+    }
 }
 bool q4k_gemm_up_format(int dt) { return dt == MOE_GGML_Q2K || dt == MOE_GGML_Q3K || dt == MOE_GGML_Q4K || dt == MOE_GGML_Q5K || dt == MOE_GGML_Q6K; }
 bool q4k_gemm_down_format(int dt) { return q4k_gemm_up_format(dt); }
 hipError_t launch_q4k_gemm_up(const ExpertParams& p_in, hipStream_t s) {
     ExpertParams p = p_in;
-    const int64_t tiles = max_gemm_tiles(p.n_slots, p.n_groups + 1, p.rb.tile_slots);
-    p.patch = patch_edge(p.F / 64, tiles);
-    dim3 grid(patch_grid(p.F / 64, tiles, p.patch));
-    if (p.dt == MOE_GGML_Q6K) launch_gemm<MOE_GGML_Q6K, 0>(p, grid, s);
-    else if (p.dt == MOE_GGML_Q5K) launch_gemm<MOE_GGML_Q5K, 0>(p, grid, s);
-    else if (p.dt == MOE_GGML_Q4K) launch_gemm<MOE_GGML_Q4K, 0>(p, grid, s);
-    else if (p.dt == MOE_GGML_Q2K) launch_gemm<MOE_GGML_Q2K, 0>(p, grid, s);
-    else if (p.dt == MOE_GGML_Q3K) launch_gemm<MOE_GGML_Q3K, 0>(p, grid, s);
+    if (p.dt == MOE_GGML_Q6K) launch_gemm<MOE_GGML_Q6K, 0>(p, s);
+    else if (p.dt == MOE_GGML_Q5K) launch_gemm<MOE_GGML_Q5K, 0>(p, s);
+    else if (p.dt == MOE_GGML_Q4K) launch_gemm<MOE_GGML_Q4K, 0>(p, s);
+    else if (p.dt == MOE_GGML_Q2K) launch_gemm<MOE_GGML_Q2K, 0>(p, s);
+    else if (p.dt == MOE_GGML_Q3K) launch_gemm<MOE_GGML_Q3K, 0>(p, s);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 hipError_t launch_q4k_gemm_down(const ExpertParams& p_in, hipStream_t s) {
     ExpertParams p = p_in;
-    const int64_t tiles = max_gemm_tiles(p.n_slots, p.n_groups + 1, p.rb.tile_slots);
-    p.patch = patch_edge(p.H / 128, tiles);
-    dim3 grid(patch_grid(p.H / 128, tiles, p.patch));
     const int dtd = p.dt_down ? p.dt_down : p.dt;
-    if (dtd == MOE_GGML_Q6K) launch_gemm<MOE_GGML_Q6K, 1>(p, grid, s);
-    else if (dtd == MOE_GGML_Q5K) launch_gemm<MOE_GGML_Q5K, 1>(p, grid, s);
-    else if (dtd == MOE_GGML_Q4K) launch_gemm<MOE_GGML_Q4K, 1>(p, grid, s);
-    else if (dtd == MOE_GGML_Q2K) launch_gemm<MOE_GGML_Q2K, 1>(p, grid, s);
-    else if (dtd == MOE_GGML_Q3K) launch_gemm<MOE_GGML_Q3K, 1>(p, grid, s);
+    if (dtd == MOE_GGML_Q6K) launch_gemm<MOE_GGML_Q6K, 1>(p, s);
+    else if (dtd == MOE_GGML_Q5K) launch_gemm<MOE_GGML_Q5K, 1>(p, s);
+    else if (dtd == MOE_GGML_Q4K) launch_gemm<MOE_GGML_Q4K, 1>(p, s);
+    else if (dtd == MOE_GGML_Q2K) launch_gemm<MOE_GGML_Q2K, 1>(p, s);
+    else if (dtd == MOE_GGML_Q3K) launch_gemm<MOE_GGML_Q3K, 1>(p, s);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
