@@ -17,7 +17,8 @@
 // different scales, so each is issued twice, with the weight operand of the lane groups that hold the
 // other sub-block zeroed; the codes stay unsigned (0..63) and the -32 is taken out through the
 // activations' 16-element sums: sum_j sc_j * bsum_j is one exact f16 MFMA (|bsum| <= 2032,
-// |sc| <= 128, the sum of sixteen products stays below 2^24).
+// |sc| <= 128, the sum of sixteen products stays below 2^24).  With two slot tiles per pass the
+// scales go into the weight operand instead (q6k_planes_of).
 //
 //   q4k_up_kernel    h[slot, f] = silu(W1 x) * (W3 x) for a 256-row block of F, then the block is
 //                    quantised to Q8K in the epilogue (Mlp::forward, quantized_llama.rs:124-131;
@@ -28,6 +29,7 @@
 
 #include "act_quant.hpp"
 #include "kernels.hpp"
+#include "planes.hpp"
 #include "slots.hpp"
 
 namespace moe {
@@ -360,6 +362,57 @@ __device__ inline void q6k_mac(const Q6KTile& w, const Q8KOperand& A, const floa
     }
 }
 
+// The same contribution with the scales inside the weight operand, for workgroups that carry two slot tiles: the scaled
+// codes W = sc * (code - 32) as two signed byte planes, W = 256 hi + lo (planes.hpp), eight v_mfma_i32_16x16x64_i8 per
+// 16-slot operand, and an unpacking (~185 vector instructions per tile) that serves both operands.  These kernels are bound
+// by vector instructions: ~225 per tile against ~430 for q6k_mac twice (32000 x 4096 at 32 rows 42.8 -> 35.0 us per call,
+// 4096 x 4096 at 20 rows 18.9 -> 12.8, an all-Q6_K Mixtral layer at 100 tokens 389 -> 268).  With one operand the two
+// count alike and measured alike (8 tokens 198 / 199 us).
+struct Q6KPlanes {
+    v4i lo[4], hi[4];
+    float d;
+};
+__device__ inline Q6KPlanes q6k_planes_of(const Q6KTile& w, int g) {
+    const uint32_t M4 = 0x0f0f0f0fu, M2H = 0x30303030u;
+    Q6KPlanes pl;
+    pl.d = __half2float(__ushort_as_half((unsigned short)w.d));
+    const uint32_t sel = (uint32_t)(g >> 1) * 8u;   // lane groups 0,1 carry elements 0..15 of a 32-element stretch, 2,3 elements 16..31
+    const uint32_t qw[8] = {w.q0.x, w.q0.y, w.q0.z, w.q0.w, w.q1.x, w.q1.y, w.q1.z, w.q1.w};
+    const uint32_t hw[4] = {w.qh.x, w.qh.y, w.qh.z, w.qh.w};
+    const uint32_t sw[4] = {w.sc.x, w.sc.y, w.sc.z, w.sc.w};
+#pragma unroll
+    for (int P = 0; P < 4; P++) {
+        const uint32_t wx = qw[2 * P], wy = qw[2 * P + 1], h = hw[P];
+        const int sa = __builtin_amdgcn_sbfe(sw[P], sel, 8), sb = __builtin_amdgcn_sbfe(sw[P], sel + 16u, 8);
+        const uint32_t sa2 = __builtin_amdgcn_perm((uint32_t)sa, (uint32_t)sa, 0x05040100u);
+        const uint32_t sb2 = __builtin_amdgcn_perm((uint32_t)sb, (uint32_t)sb, 0x05040100u);
+        const uint32_t aa2 = pk_mad_u16(sa2, 0xffe0ffe0u, 0x00800080u), ab2 = pk_mad_u16(sb2, 0xffe0ffe0u, 0x00800080u);
+        int l0, l1, l2, l3, h0, h1, h2, h3;
+        q6k_planes((wx & M4) | ((h << 4) & M2H), sa2, aa2, l0, h0);
+        q6k_planes((wy & M4) | ((h << 2) & M2H), sa2, aa2, l1, h1);
+        q6k_planes(((wx >> 4) & M4) | (h & M2H), sb2, ab2, l2, h2);
+        q6k_planes(((wy >> 4) & M4) | ((h >> 2) & M2H), sb2, ab2, l3, h3);
+        pl.lo[P] = v4i{l0, l1, l2, l3};
+        pl.hi[P] = v4i{h0, h1, h2, h3};
+    }
+    return pl;
+}
+__device__ inline void q6k_mac_planes(const Q6KPlanes& pl, const Q8KOperand& A, const float yd[4], float acc[4]) {
+    const v4i zero = {0, 0, 0, 0};
+    v4i p_lo = zero, p_hi = zero;
+#pragma unroll
+    for (int P = 0; P < 4; P++) {
+        const v4i a = {(int)A.a[P].x, (int)A.a[P].y, (int)A.a[P].z, (int)A.a[P].w};
+        p_lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl.lo[P], p_lo, 0, 0, 0);
+        p_hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl.hi[P], p_hi, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int tot = (p_hi[i] << 8) + p_lo[i];   // exact: |tot| < 2^28
+        acc[i] += (pl.d * yd[i]) * (float)tot;
+    }
+}
+
 // Q3K (BlockQ3K::vec_dot, k_quants.rs:927-1045): d * y.d * sum_j (sc_j - 32) * (code_j . q8_j), codes -4..3, one
 // signed 6-bit scale per 16 elements: the Q6K scheme with 3-bit unsigned codes (code + 4 = low two bits |
 // high bit << 2) and the offset -4 taken out through the activations' 16-element sums.
@@ -478,6 +531,14 @@ struct FmtQ6K {
     static __device__ inline Tile load(const uint8_t* tile, int lane) { return load_q6k_tile(tile, lane); }
     static __device__ inline const Tile& prepare(const Tile& w, int) { return w; }
     static __device__ inline void mac(const Tile& w, const Q8KOperand& A, const float yd[4], int g, float acc[4]) { q6k_mac(w, A, yd, g, acc); }
+};
+// Q6K with the scales inside the weight operand: for two slot tiles per pass
+struct FmtQ6KP {
+    typedef Q6KTile Tile;
+    static constexpr int TILE_BYTES = Q6K_TILE_BYTES;
+    static __device__ inline Tile load(const uint8_t* tile, int lane) { return load_q6k_tile(tile, lane); }
+    static __device__ inline Q6KPlanes prepare(const Tile& w, int g) { return q6k_planes_of(w, g); }
+    static __device__ inline void mac(const Q6KPlanes& pl, const Q8KOperand& A, const float yd[4], int, float acc[4]) { q6k_mac_planes(pl, A, yd, acc); }
 };
 
 // One wave, NT weight tiles per super-block (tp[0..NT), each walking along K), TT 16-slot operand
@@ -835,10 +896,10 @@ DEF_DOWN(q5k_down_t2, FmtQ5K, 2, 4, 2, 2)
 // registers of a two-waves-per-SIMD launch, and four slot tiles per pass would spill: two at most
 DEF_UP(q6k_up_t1, FmtQ6K, 1, 4, 2, 2)
 DEF_UP_NARROW(q6k_up_t1_narrow, FmtQ6K, 4, 2, 2)
-DEF_UP(q6k_up_t2, FmtQ6K, 2, 4, 2, 2)
+DEF_UP(q6k_up_t2, FmtQ6KP, 2, 4, 2, 2)
 DEF_DOWN(q6k_down_t1, FmtQ6K, 1, 4, 2, 2)
 DEF_DOWN_NARROW(q6k_down_t1_narrow, FmtQ6K, 8, 2, 2)
-DEF_DOWN(q6k_down_t2, FmtQ6K, 2, 4, 2, 2)
+DEF_DOWN(q6k_down_t2, FmtQ6KP, 2, 4, 2, 2)
 
 DEF_DOWN_FINE(q4k_down_t1_fine, FmtQ4K, 1, 4, 4, 3)
 DEF_DOWN_FINE(q4k_down_t2_fine, FmtQ4KP, 2, 4, 4, 2)
@@ -850,7 +911,7 @@ DEF_DOWN_FINE(q3k_down_t2_fine, FmtQ3K, 2, 4, 4, 2)
 DEF_DOWN_FINE(q5k_down_t1_fine, FmtQ5K, 1, 4, 4, 3)
 DEF_DOWN_FINE(q5k_down_t2_fine, FmtQ5K, 2, 4, 4, 2)
 DEF_DOWN_FINE(q6k_down_t1_fine, FmtQ6K, 1, 4, 4, 2)
-DEF_DOWN_FINE(q6k_down_t2_fine, FmtQ6K, 2, 4, 4, 2)
+DEF_DOWN_FINE(q6k_down_t2_fine, FmtQ6KP, 2, 4, 4, 2)
 
 // ---------------------------------------------------------------------------------------------
 // Dense matrix times a few rows (single-stream decoding: attention projections, output head) in one launch: the rows
