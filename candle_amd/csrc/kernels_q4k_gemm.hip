@@ -25,7 +25,7 @@
 // issued a few at a time behind the operands (in one go at the top they held each wave up for 1650 to 4700 of 9000 cycles).
 // Up launch, 4096 tokens at the Mixtral shape: one operand per wave, four waves per SIMD 2.26 ms, this kernel 1.97 ms;
 // the same with 32x32x32 MFMAs and no overlap in the wave 2.3 ms.  Operands beyond a short tile's list are neither
-// fetched nor multiplied (the K loop exists for 8, 6, 4 and 2 of them).
+// fetched nor multiplied (the K loop exists for each number of them).
 //
 // Q6K weights (the w2 of mixed files) take the same kernel for the down projection.  BlockQ6K::vec_dot
 // (k_quants.rs:1613-1671) is d * y.d * sum_j sc_j * ((code_j - 32) . q8_j) with an i8 scale per 16 elements; the
@@ -516,10 +516,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
             __syncthreads();
         }
     };
-    if (live > NOP * 3 / 4) run(std::integral_constant<int, NOP>{});
-    else if (live > NOP / 2) run(std::integral_constant<int, NOP * 3 / 4>{});
-    else if (NOP == 4 || live > NOP / 4) run(std::integral_constant<int, NOP / 2>{});
-    else run(std::integral_constant<int, NOP / 4>{});
+    static_for<1, NOP + 1>([&](auto lv_tag) {
+        constexpr int LV = decltype(lv_tag)::value;
+        if (live == LV) run(lv_tag);
+    });
 
     // epilogue: lane holds weight row n = lane%16 of both operands and slots 16 o + 4 (lane/16) + i
     const int n = lane & 15, g = lane >> 4;
@@ -544,10 +544,12 @@ template <int FMT, int MODE>
 static void launch_gemm(ExpertParams& p, hipStream_t s) {
     const int64_t tiles = max_gemm_tiles(p.n_slots, p.n_groups + 1, p.rb.tile_slots);
     const int64_t rows = MODE == 0 ? 2 * (int64_t)p.F : p.H;
-    // Workgroups of eight waves (256 weight rows) fetch an activation tile half as often as those of four.  (Mixtral shape, Q4_K,
-    // us, eight / four waves: 301 tokens 467 / 519, 4096 tokens 3210 / 3282; 777 rows x 4096 x 4096, 208 / 416 workgroups of
-    // 64 slots: 54 / 58.)  A grid that would leave half of the CUs without one takes the four-wave ones.
-    const bool wide = rows % 256 == 0 && rows / 256 * tiles >= 128;
+    // Workgroups of eight waves (256 weight rows, one per CU) fetch an activation tile half as often as those of four (two
+    // per CU), but a grid of them that fills little more than half of the CUs loses more than that.  (Mixtral shape, Q4_K / Q6_K
+    // down, us per step with eight / four waves in the down kernel: 301 tokens, 144 workgroups of eight waves 428 / 386; 600
+    // tokens, ~220 of them 624 / 644; in the up kernel, ~970 of them 428 / 441; 777 rows x 4096 x 4096, 208 of them 56 / 58.)
+    // The tiles are estimated: half a tile per group beyond the full ones.
+    const bool wide = rows % 256 == 0 && rows / 256 * (p.n_slots / p.rb.tile_slots + (p.n_groups + 1) / 2) >= 170;
     const int64_t n_rb = rows / (wide ? 256 : 128);
     p.patch = patch_edge(n_rb, tiles);
     const dim3 grid(patch_grid(n_rb, tiles, p.patch));

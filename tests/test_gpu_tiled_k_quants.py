@@ -27,7 +27,7 @@ def check(dt, n, k, rows):
 
 
 @pytest.mark.parametrize("dt", K_QUANTS)
-@pytest.mark.parametrize("n", [12288, 12416])
+@pytest.mark.parametrize("n", [24576, 12416])
 def test_tiles_of_64_rows(dt, n):
     check(dt, n, 512, (96, 97, 112, 128, 129, 161, 177))
 
