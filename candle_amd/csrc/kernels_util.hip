@@ -446,40 +446,42 @@ __global__ void dequant_tiled_kernel(int dt, const uint8_t* tiled, float* out, i
 }
 
 // ------------------------------------------------------------------ activation quantiser on plain rows
+// Q8K: the rows are one run of 256-element blocks, in memory and in every part of the ActBuf, so block n of the run is all a
+// wave has to know.  NQ consecutive blocks per wave, side by side (their loads, wave reductions and divisions overlap):
+// four where there are waves enough, fewer for a few rows.  Bound by HBM at thousands of rows (8192 x 14336: 115 -> 103 us, 5.7 TB/s), by the
+// latency of one load, reduction and division below.  Dealing a row's blocks to the waves of a few workgroups left half of
+// the four places empty at 777 x 4096 (9.0 -> 7.0 us) and 40 % at 602 x 14336 (15.9 -> 13.0 us).
+template <int NQ>
+__global__ __launch_bounds__(256) void quantize_q8k_rows_kernel(const float* x, int64_t n_blocks, ActBuf out) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t b0 = ((int64_t)blockIdx.x * 4 + wave) * NQ;
+    if (b0 >= n_blocks) return;
+    float4 v[NQ];
+    bool valid[NQ];
+    int8_t* qs_out[NQ];
+    float* d_out[NQ];
+    __half* bs_out[NQ];
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+        valid[n] = b0 + n < n_blocks;
+        const int64_t b = valid[n] ? b0 + n : b0;
+        v[n] = *reinterpret_cast<const float4*>(x + b * 256 + lane * 4);
+        qs_out[n] = out.qs + b * 256;
+        d_out[n] = out.d + b;
+        bs_out[n] = reinterpret_cast<__half*>(out.bsum) + b * 16;
+    }
+    quantize_q8k_blocks<NQ>(v, valid, lane, qs_out, d_out, bs_out);
+}
 template <int VDT>
-__global__ __launch_bounds__(256) void quantize_rows_kernel(const float* x, int64_t rows, int k, ActBuf out) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__global__ __launch_bounds__(256) void quantize_rows_kernel(const float* x, int k, ActBuf out) {
     const int64_t row = blockIdx.x;
     const float* xr = x + row * k;
-    if (VDT == MOE_GGML_Q8K) {
-        // blocks of a row are dealt to the waves of gridDim.y workgroups (few rows: many workgroups per row)
-        // (four blocks of a wave side by side: their loads, wave reductions and divisions overlap)
-        const int nb = k / 256;
-        constexpr int NQ = 4;
-        const int stride = 4 * gridDim.y;
-        for (int b0 = blockIdx.y * 4 + wave; b0 < nb; b0 += NQ * stride) {
-            float4 v[NQ];
-            bool valid[NQ];
-            int8_t* qs_out[NQ];
-            float* d_out[NQ];
-            __half* bs_out[NQ];
-#pragma unroll
-            for (int n = 0; n < NQ; n++) {
-                valid[n] = b0 + n * stride < nb;
-                const int b = valid[n] ? b0 + n * stride : b0;
-                v[n] = *reinterpret_cast<const float4*>(xr + b * 256 + lane * 4);
-                qs_out[n] = out.qs + row * k + b * 256;
-                d_out[n] = out.d + row * nb + b;
-                bs_out[n] = reinterpret_cast<__half*>(out.bsum) + (row * nb + b) * 16;
-            }
-            quantize_q8k_blocks<NQ>(v, valid, lane, qs_out, d_out, bs_out);
-        }
-    } else {
-        const int nb = k / 32;
-        for (int h = blockIdx.y * 256 + tid; h < k; h += 256 * gridDim.y)
-            quantize_q8_0_block(VDT, xr[h], lane, out.qs + row * k + h, out.d + row * nb + h / 32,
-                                reinterpret_cast<int32_t*>(out.bsum) + row * nb + h / 32);
-    }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int nb = k / 32;
+    for (int h = blockIdx.y * 256 + tid; h < k; h += 256 * gridDim.y)
+        quantize_q8_0_block(VDT, xr[h], lane, out.qs + row * k + h, out.d + row * nb + h / 32,
+                            reinterpret_cast<int32_t*>(out.bsum) + row * nb + h / 32);
 }
 
 // ActBuf -> the reference's block structs (BlockQ8K 292 B: d f32, qs[256], bsums i16[16];
@@ -555,14 +557,20 @@ hipError_t launch_dequant_std(int dt, const uint8_t* blocks, float* out, int64_t
 
 hipError_t launch_quantize_rows(int vdt, const float* x, int64_t rows, int k, const ActBuf& out, hipStream_t s) {
     if (rows == 0) return hipSuccess;
-    const int64_t per_row = vdt == MOE_GGML_Q8K ? (k / 256 + 3) / 4 : (k + 255) / 256;   // workgroups that have a share of a row
+    if (vdt == MOE_GGML_Q8K) {
+        // eight waves per CU before a wave takes more than one block, sixteen before it takes four
+        const int64_t n = rows * (k / 256);
+        if (n >= 4 * 4096) hipLaunchKernelGGL(quantize_q8k_rows_kernel<4>, dim3(nblk(n, 16)), dim3(256), 0, s, x, n, out);
+        else if (n >= 2 * 2048) hipLaunchKernelGGL(quantize_q8k_rows_kernel<2>, dim3(nblk(n, 8)), dim3(256), 0, s, x, n, out);
+        else hipLaunchKernelGGL(quantize_q8k_rows_kernel<1>, dim3(nblk(n, 4)), dim3(256), 0, s, x, n, out);
+        return hipGetLastError();
+    }
+    const int64_t per_row = (k + 255) / 256;   // workgroups that have a share of a row
     const unsigned split = (unsigned)std::max<int64_t>(1, std::min<int64_t>(per_row, 2048 / rows));
-    if (vdt == MOE_GGML_Q8K)
-        hipLaunchKernelGGL(quantize_rows_kernel<MOE_GGML_Q8K>, dim3((unsigned)rows, split), dim3(256), 0, s, x, rows, k, out);
-    else if (vdt == MOE_GGML_Q8_1)
-        hipLaunchKernelGGL(quantize_rows_kernel<MOE_GGML_Q8_1>, dim3((unsigned)rows, split), dim3(256), 0, s, x, rows, k, out);
+    if (vdt == MOE_GGML_Q8_1)
+        hipLaunchKernelGGL(quantize_rows_kernel<MOE_GGML_Q8_1>, dim3((unsigned)rows, split), dim3(256), 0, s, x, k, out);
     else
-        hipLaunchKernelGGL(quantize_rows_kernel<MOE_GGML_Q8_0>, dim3((unsigned)rows, split), dim3(256), 0, s, x, rows, k, out);
+        hipLaunchKernelGGL(quantize_rows_kernel<MOE_GGML_Q8_0>, dim3((unsigned)rows, split), dim3(256), 0, s, x, k, out);
     return hipGetLastError();
 }
 
