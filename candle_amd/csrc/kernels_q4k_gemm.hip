@@ -23,7 +23,7 @@
 // takes two waves per SIMD (256 registers), too few to cover each other, so a wave overlaps its own work: the results of
 // operand o - 1 are added up between the matrix instructions of operand o, and the next super-block's transfers are
 // issued a few at a time behind the operands (in one go at the top they held each wave up for 1650 to 4700 of 9000 cycles).
-// Up launch, 4096 tokens at the Mixtral shape: one operand per wave, four waves per SIMD 2.26 ms, this kernel 1.97 ms;
+// Up launch, 4096 tokens at the Mixtral shape: one operand per wave, four waves per SIMD 2.23-2.28 ms, this kernel 2.00-2.12 ms;
 // the same with 32x32x32 MFMAs and no overlap in the wave 2.3 ms.  Operands beyond a short tile's list are neither
 // fetched nor multiplied (the K loop exists for each number of them).
 //
