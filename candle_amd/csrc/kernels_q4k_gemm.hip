@@ -38,6 +38,7 @@
 // eight; the minimums leave through the sixteen block sums as for Q4K.
 #include <type_traits>
 #include "act_quant.hpp"
+#include "gemm_plan.hpp"
 #include "kernels.hpp"
 #include "planes.hpp"
 
@@ -544,18 +545,18 @@ template <int FMT, int MODE>
 static void launch_gemm(ExpertParams& p, hipStream_t s) {
     const int64_t tiles = max_gemm_tiles(p.n_slots, p.n_groups + 1, p.rb.tile_slots);
     const int64_t rows = MODE == 0 ? 2 * (int64_t)p.F : p.H;
-    // Workgroups of eight waves (256 weight rows, one per CU) fetch an activation tile half as often as those of four (two
-    // per CU), but a grid of them that fills little more than half of the CUs loses more than that.  (Mixtral shape, Q4_K / Q6_K
-    // down, us per step with eight / four waves in the down kernel: 301 tokens, 144 workgroups of eight waves 428 / 386; 600
-    // tokens, ~220 of them 624 / 644; in the up kernel, ~970 of them 428 / 441; 777 rows x 4096 x 4096, 208 of them 56 / 58.)
-    // The tiles are estimated: half a tile per group beyond the full ones.
-    const bool wide = rows % 256 == 0 && rows / 256 * (p.n_slots / p.rb.tile_slots + (p.n_groups + 1) / 2) >= 170;
+    const bool wide = gemm_wide(MODE == 0, rows, p.n_slots, p.n_groups, p.rb.tile_slots);
     const int64_t n_rb = rows / (wide ? 256 : 128);
     p.patch = patch_edge(n_rb, tiles);
     const dim3 grid(patch_grid(n_rb, tiles, p.patch));
     if (p.rb.tile_slots == 64) {
-        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8>), grid, dim3(512), 0, s, p);
-        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4>), grid, dim3(256), 0, s, p);
+        if constexpr (MODE == 1) {
+            if (wide) {
+                hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8>), grid, dim3(512), 0, s, p);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4>), grid, dim3(256), 0, s, p);
     } else {
         if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 8>), grid, dim3(512), 0, s, p);
         else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 4>), grid, dim3(256), 0, s, p);
