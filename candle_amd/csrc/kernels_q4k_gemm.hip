@@ -26,6 +26,9 @@
 // Up launch, 4096 tokens at the Mixtral shape: one operand per wave, four waves per SIMD 2.23-2.28 ms, this kernel 2.00-2.12 ms;
 // the same with 32x32x32 MFMAs and no overlap in the wave 2.3 ms.  Operands beyond a short tile's list are neither
 // fetched nor multiplied (the K loop exists for each number of them).
+// Down launches of the formats that unpack longest in tiles of 64 slots run one operand per wave at four waves per SIMD
+// (launch_gemm).  Registers: 164 to 254 with two operands (Q5K at 128 slots: 256, one to three of them spilled outside the K
+// loop), 122 to 126 with one.
 //
 // Q6K weights (the w2 of mixed files) take the same kernel for the down projection.  BlockQ6K::vec_dot
 // (k_quants.rs:1613-1671) is d * y.d * sum_j sc_j * ((code_j - 32) . q8_j) with an i8 scale per 16 elements; the
@@ -344,16 +347,17 @@ __device__ __forceinline__ BPlanes b_planes(const BRegs& r, int lane) {
     else return b_prepare(r, lane);
 }
 
-// The matrix results of one 16-slot operand against the wave's two 16-row weight operands, on their way to the sums.
+// The matrix results of one 16-slot operand against the wave's J 16-row weight operands, on their way to the sums.
+template <int J>
 struct OperandAcc {
-    v4i lo[2], hi[2];
-    v4f dm[2], yd;
+    v4i lo[J], hi[J];
+    v4f dm[J], yd;
 };
-// Adds result i (slot 16 o + 4 g + i, weight rows n = lane%16 of both operands) of a super-block to the sums.
-template <int FMT>
-__device__ __forceinline__ void gemm_result(const BPlanes (&B)[2], const OperandAcc& A, int i, v4f (&facc)[2]) {
+// Adds result i (slot 16 o + 4 g + i, weight rows n = lane%16 of its operands) of a super-block to the sums.
+template <int FMT, int J>
+__device__ __forceinline__ void gemm_result(const BPlanes (&B)[J], const OperandAcc<J>& A, int i, v4f (&facc)[J]) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+    for (int j = 0; j < J; j++) {
         if constexpr (FMT == MOE_GGML_Q6K || FMT == MOE_GGML_Q3K) {
             const int isum = (A.hi[j][i] << 8) + A.lo[j][i];
             facc[j][i] = __builtin_fmaf(B[j].d * A.yd[i], (float)isum, facc[j][i]);
@@ -376,14 +380,14 @@ __device__ __forceinline__ void gemm_result(const BPlanes (&B)[2], const Operand
 __device__ __forceinline__ v4i operand_piece(const uint8_t* q, int o, int P, int lane) {
     return *reinterpret_cast<const v4i*>(q + o * 4096 + P * 1024 + lane * 16);
 }
-// One super-block of the wave's 32 weight rows against operands O, O + 1, ... of the staged tile.  While the matrix
+// One super-block of the wave's 16 J weight rows against operands O, O + 1, ... of the staged tile.  While the matrix
 // instructions of an operand run, the wave's vector instructions add up the results of the operand before it (`prev`).
-template <int FMT, int NOP, int LV, int O, class Fill>
-__device__ __forceinline__ void gemm_operands(const BPlanes (&B)[2], const GemmLds<NOP>& L, int buf, int lane, v4i (&a)[4], OperandAcc& prev,
-                                              v4f (&facc)[NOP][2], const Fill& fill) {
+template <int FMT, int NOP, int LV, int O, int J, class Fill>
+__device__ __forceinline__ void gemm_operands(const BPlanes (&B)[J], const GemmLds<NOP>& L, int buf, int lane, v4i (&a)[4], OperandAcc<J>& prev,
+                                              v4f (&facc)[NOP][J], const Fill& fill) {
     const int m = lane & 15, g = lane >> 4;
     const v4i zero4 = {0, 0, 0, 0};
-    OperandAcc cur;
+    OperandAcc<J> cur;
     v4h mA;
     if constexpr (FMT != MOE_GGML_Q6K && FMT != MOE_GGML_Q3K) mA = *reinterpret_cast<const v4h*>(&L.bs[buf][O][g >> 1][m][(g & 1) * 4]);
     cur.yd = *reinterpret_cast<const v4f*>(&L.yd[buf][O * 16 + g * 4]);
@@ -391,17 +395,19 @@ __device__ __forceinline__ void gemm_operands(const BPlanes (&B)[2], const GemmL
     for (int P = 0; P < 4; P++) {
         const v4i x = a[P];
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < J; j++) {
             cur.lo[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, B[j].lo[P], P == 0 ? zero4 : cur.lo[j], 0, 0, 0);
             if constexpr (FMT != MOE_GGML_Q2K) cur.hi[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, B[j].hi[P], P == 0 ? zero4 : cur.hi[j], 0, 0, 0);
         }
         if constexpr (O + 1 < LV) a[P] = operand_piece(L.q[buf], O + 1, P, lane);
-        if constexpr (O > 0) gemm_result<FMT>(B, prev, P, facc[O - 1]);
+        if constexpr (O > 0) gemm_result<FMT, J>(B, prev, P, facc[O - 1]);
         // order: a matrix instruction (mask 0x8), three vector instructions (0x2), and so on
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+        if constexpr (J == 2) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+        }
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
@@ -412,26 +418,27 @@ __device__ __forceinline__ void gemm_operands(const BPlanes (&B)[2], const GemmL
     if constexpr (FMT != MOE_GGML_Q6K && FMT != MOE_GGML_Q3K) {
         const v4f zf = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 2; j++) cur.dm[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(mA, B[j].mB, zf, 0, 0, 0);
+        for (int j = 0; j < J; j++) cur.dm[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(mA, B[j].mB, zf, 0, 0, 0);
     }
     prev = cur;
     if constexpr (O + 1 < LV) {
-        gemm_operands<FMT, NOP, LV, O + 1>(B, L, buf, lane, a, prev, facc, fill);
+        gemm_operands<FMT, NOP, LV, O + 1, J>(B, L, buf, lane, a, prev, facc, fill);
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) gemm_result<FMT>(B, prev, i, facc[O]);
+    for (int i = 0; i < 4; i++) gemm_result<FMT, J>(B, prev, i, facc[O]);
 }
 
 __device__ __forceinline__ float silu_gemm(float v) { return v / (1.0f + __expf(-v)); }
 
 // ---------------------------------------------------------------------------------------------
-// Two 16-row weight operands per wave, NW waves per workgroup, two waves per SIMD; a tile of NOP*16 slots.
-// MODE 0: up   -- a wave carries 16 rows of w1 and the same 16 rows of w3 and writes h = silu(a) * b (f32).
-// MODE 1: down -- 32 rows of w2 per wave; writes yw.
+// J 16-row weight operands per wave, NW waves per workgroup, 4 / J waves per SIMD; a tile of NOP*16 slots.
+// MODE 0: up   -- a wave carries 16 rows of w1 and the same 16 rows of w3 (J = 2) and writes h = silu(a) * b (f32).
+// MODE 1: down -- 16 J rows of w2 per wave; writes yw.
 // FMT: the weights' format (Q2K ... Q6K).
-template <int FMT, int MODE, int NOP, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void q4k_gemm_kernel(ExpertParams p) {
+template <int FMT, int MODE, int NOP, int NW, int J>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4 / J, 4 / J))) void q4k_gemm_kernel(ExpertParams p) {
+    static_assert(J == 2 || (J == 1 && MODE == 1), "the up projection takes w1 and w3 side by side");
     static_assert(FMT == MOE_GGML_Q2K || FMT == MOE_GGML_Q3K || FMT == MOE_GGML_Q4K || FMT == MOE_GGML_Q5K || FMT == MOE_GGML_Q6K, "formats of the tiled kernel");
     constexpr int NB = NOP * 4 / NW;
     constexpr int TILE_BYTES = FMT == MOE_GGML_Q6K ? Q6K_TILE_BYTES : FMT == MOE_GGML_Q5K ? Q5K_TILE_BYTES : FMT == MOE_GGML_Q2K ? Q2K_TILE_BYTES : FMT == MOE_GGML_Q3K ? Q3K_TILE_BYTES : Q4K_TILE_BYTES;
@@ -441,7 +448,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n_tiles = p.rb.tile_tab[0];
     // workgroup -> (row block, slot tile), in patches per XCD (patch_position)
-    const int n_rb = MODE == 0 ? p.F / (16 * NW) : p.H / (32 * NW);
+    const int n_rb = MODE == 0 ? p.F / (16 * NW) : p.H / (16 * J * NW);
     const PatchPos pos = patch_position((int)blockIdx.x, n_rb, p.patch);
     const int rblk = pos.rblk, tile = pos.tile;
     if (tile >= n_tiles || rblk >= n_rb) return;
@@ -469,24 +476,28 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
     // weight operands of this wave
     const GroupWeights gw = p.groups[grp];
-    const int row0 = (rblk * NW + wave) * (MODE == 0 ? 16 : 32);
-    const uint8_t* wp[2];
+    const int row0 = (rblk * NW + wave) * (MODE == 0 ? 16 : 16 * J);
+    const uint8_t* wp[J];
     if (MODE == 0) {
         wp[0] = gw.w1 + (size_t)(row0 / 16) * TILE_BYTES;
-        wp[1] = gw.w3 + (size_t)(row0 / 16) * TILE_BYTES;
+        wp[J - 1] = gw.w3 + (size_t)(row0 / 16) * TILE_BYTES;
     } else {
-        wp[0] = gw.w2 + (size_t)(row0 / 16) * TILE_BYTES;
-        wp[1] = wp[0] + TILE_BYTES;
-    }
-    v4f facc[NOP][2];
 #pragma unroll
-    for (int o = 0; o < NOP; o++) facc[o][0] = facc[o][1] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < J; j++) wp[j] = gw.w2 + (size_t)(row0 / 16 + j) * TILE_BYTES;
+    }
+    v4f facc[NOP][J];
+#pragma unroll
+    for (int o = 0; o < NOP; o++)
+#pragma unroll
+        for (int j = 0; j < J; j++) facc[o][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
     // operands of the tile that hold slots of the list: a short tile's others are neither fetched nor multiplied
     const int live = __builtin_amdgcn_readfirstlane(min(NOP, (n_g - pos0 + 15) >> 4));
     auto stage = [&](auto I, int sb, int buf) { stage_piece<decltype(I)::value, kSums, NOP, NB>(ab, rows, sb, L, buf, wave, live); };
     static_for<0, NB + 2>([&](auto I) { stage(I, 0, 0); });
-    BRegs raw[2] = {b_load<FMT>(wp[0], lane), b_load<FMT>(wp[1], lane)};
+    BRegs raw[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) raw[j] = b_load<FMT>(wp[j], lane);
     wait_all_loads();
     __syncthreads();
     // the K loop over LV operands
@@ -495,19 +506,22 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int sb = 0; sb < nsb; sb++) {
             const int buf = sb & 1, nb = buf ^ 1;
             const int sbn = sb + 1 < nsb ? sb + 1 : sb;
-            const BPlanes B[2] = {b_planes<FMT>(raw[0], lane), b_planes<FMT>(raw[1], lane)};
+            BPlanes B[J];
+#pragma unroll
+            for (int j = 0; j < J; j++) B[j] = b_planes<FMT>(raw[j], lane);
             // (for the sake of the registers the next weights are requested after this super-block's are unpacked)
             __builtin_amdgcn_sched_barrier(0);
             v4i a[4];
 #pragma unroll
             for (int P = 0; P < 4; P++) a[P] = operand_piece(L.q[buf], 0, P, lane);
-            OperandAcc prev;
+            OperandAcc<J> prev;
             // The next super-block's weights and activations are requested while the operands are multiplied, a few requests at a
             // time: issued in one go they fill the CU's memory queue and the wave stands still for a thousand cycles and more.
-            gemm_operands<FMT, NOP, LV, 0>(B, L, buf, lane, a, prev, facc, [&](auto o_tag) {
+            gemm_operands<FMT, NOP, LV, 0, J>(B, L, buf, lane, a, prev, facc, [&](auto o_tag) {
                 constexpr int O = decltype(o_tag)::value;
-                if constexpr (O == 0) raw[0] = b_load<FMT>(wp[0] + (size_t)sbn * sb_stride, lane);
-                if constexpr (O == (LV > 2 ? 1 : 0)) raw[1] = b_load<FMT>(wp[1] + (size_t)sbn * sb_stride, lane);
+                // (four waves per SIMD: a format with block sums has registers for the next weights behind its last operand only)
+                if constexpr (O == (J == 1 && kSums ? LV - 1 : 0)) raw[0] = b_load<FMT>(wp[0] + (size_t)sbn * sb_stride, lane);
+                if constexpr (J == 2 && O == (LV > 2 ? 1 : 0)) raw[J - 1] = b_load<FMT>(wp[J - 1] + (size_t)sbn * sb_stride, lane);
                 constexpr int FIRST = LV > 2 ? 1 : 0, SPAN = LV > 4 ? LV - 3 : 1;
                 static_for<0, NB + 2>([&](auto I) {
                     if constexpr (FIRST + decltype(I)::value * SPAN / (NB + 2) == O) stage(I, sbn, nb);
@@ -522,7 +536,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         if (live == LV) run(lv_tag);
     });
 
-    // epilogue: lane holds weight row n = lane%16 of both operands and slots 16 o + 4 (lane/16) + i
+    // epilogue: lane holds weight row n = lane%16 of its operands and slots 16 o + 4 (lane/16) + i
     const int n = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int o = 0; o < NOP; o++)
@@ -532,11 +546,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
             if (pos >= n_g) continue;
             const int slot = s_begin + pos;
             if (MODE == 0) {
-                p.hbuf[(int64_t)(slot - p.slot_origin) * p.F + row0 + n] = silu_gemm(facc[o][0][i]) * facc[o][1][i];
+                p.hbuf[(int64_t)(slot - p.slot_origin) * p.F + row0 + n] = silu_gemm(facc[o][0][i]) * facc[o][J - 1][i];
             } else {
                 const float w = p.rb.perm_w[slot];
-                p.yw[(int64_t)slot * p.H + row0 + n] = facc[o][0][i] * w;
-                p.yw[(int64_t)slot * p.H + row0 + 16 + n] = facc[o][1][i] * w;
+#pragma unroll
+                for (int j = 0; j < J; j++) p.yw[(int64_t)slot * p.H + row0 + 16 * j + n] = facc[o][j][i] * w;
             }
         }
 }
@@ -545,21 +559,27 @@ template <int FMT, int MODE>
 static void launch_gemm(ExpertParams& p, hipStream_t s) {
     const int64_t tiles = max_gemm_tiles(p.n_slots, p.n_groups + 1, p.rb.tile_slots);
     const int64_t rows = MODE == 0 ? 2 * (int64_t)p.F : p.H;
-    const bool wide = gemm_wide(MODE == 0, rows, p.n_slots, p.n_groups, p.rb.tile_slots);
+    // Down launches in tiles of 64 slots whose weights take long to unpack (Q3K, Q5K, Q6K): one operand per wave, four waves per
+    // SIMD.  Their unpacking serves four operands only, and two waves cannot cover each other's: with two operands per
+    // wave they were slower at every width (us, best width / this: Q6_K 1024 x 4096 at 2048 rows 48.1 / 45.0, 4096 x 14336 at 512
+    // 126 / 115, 14336 x 4096 at 300 82.2 / 78.6, Q3_K 4096 x 4096 at 512 42.9 / 40.4, Q5_K 1024 x 4096 at 2048 50.0 / 48.6).  Q4_K and Q2_K
+    // lose by it (4096 x 4096 at 1500 rows 90 / 103 and 79 / 92).
+    constexpr bool one_operand = MODE == 1 && (FMT == MOE_GGML_Q3K || FMT == MOE_GGML_Q5K || FMT == MOE_GGML_Q6K);
+    const bool tiles64 = p.rb.tile_slots == 64;
+    const bool wide = !(one_operand && tiles64) && gemm_wide(MODE == 0, rows, p.n_slots, p.n_groups, p.rb.tile_slots);
     const int64_t n_rb = rows / (wide ? 256 : 128);
     p.patch = patch_edge(n_rb, tiles);
     const dim3 grid(patch_grid(n_rb, tiles, p.patch));
-    if (p.rb.tile_slots == 64) {
-        if constexpr (MODE == 1) {
-            if (wide) {
-                hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8>), grid, dim3(512), 0, s, p);
-                return;
-            }
-        }
-        hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4>), grid, dim3(256), 0, s, p);
+    if (!tiles64) {
+        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 8, 2>), grid, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 4, 2>), grid, dim3(256), 0, s, p);
+    } else if constexpr (one_operand) {
+        hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8, 1>), grid, dim3(512), 0, s, p);
+    } else if constexpr (MODE == 0) {
+        hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4, 2>), grid, dim3(256), 0, s, p);
     } else {
-        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 8>), grid, dim3(512), 0, s, p);
-        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 4>), grid, dim3(256), 0, s, p);
+        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8, 2>), grid, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4, 2>), grid, dim3(256), 0, s, p);
     }
 }
 bool q4k_gemm_up_format(int dt) { return dt == MOE_GGML_Q2K || dt == MOE_GGML_Q3K || dt == MOE_GGML_Q4K || dt == MOE_GGML_Q5K || dt == MOE_GGML_Q6K; }
