@@ -1,5 +1,6 @@
 // Launchers of the gfx950 kernels (definitions in the kernels_*.hip files).
 #pragma once
+#include "gemm_plan.hpp"
 #include "moe_common.hpp"
 
 namespace moe {
@@ -48,41 +49,6 @@ struct RouteBufs {
 constexpr int DISPATCH_MAX_WGS = 32;      // workgroups of a dispatch pass in two launches
 constexpr int DISPATCH_COUNT_STRIDE = 256;  // ints per workgroup in wg_counts: the largest expert count
 constexpr int DIRECT_MAX_SLOTS = 1024;  // largest T*k (and T) served without a dispatch pass
-constexpr int GEMM_MIN_TILE_SLOTS = 64;  // smallest tile of the tiled expert kernels
-inline int64_t max_gemm_tiles(int64_t slots, int64_t groups, int tile_slots = GEMM_MIN_TILE_SLOTS) { return slots / tile_slots + groups + 1; }
-
-// Tiled kernels: workgroup id -> (row block, slot tile).  Hardware hands consecutive workgroup ids to the eight XCDs in
-// turn, each with its own L2; the ids that land on one XCD are walked in patches of edge x edge (row blocks x tiles), so
-// that the workgroups an XCD runs at a time share their weight rows and their activation tiles through that L2.  The
-// edge is 8 when that still gives every XCD at least two patches, else 4 or 2: a grid of a few hundred workgroups cut
-// into 8 x 8 patches would leave XCDs without work.
-struct PatchPos { int rblk, tile; };
-// `patch` = rows edge + 256 * tiles edge (a tiles edge of 0: a square patch)
-__host__ __device__ inline PatchPos patch_position(int block, int n_rb, int patch) {
-    const int er = patch & 255, et = (patch >> 8) ? (patch >> 8) : er;
-    const int per = er * et, RG = (n_rb + er - 1) / er;
-    const int xcd = block & 7, q = block >> 3;
-    const int st = (q / per) * 8 + xcd, within = q % per;
-    return PatchPos{(st % RG) * er + within % er, (st / RG) * et + within / er};
-}
-inline int patch_edge(int64_t n_rb, int64_t tiles) {
-    for (int e = 8; e > 2; e >>= 1)
-        if (((n_rb + e - 1) / e) * ((tiles + e - 1) / e) >= 16) return e;
-    return 2;
-}
-// One group of a few tiles (the always-on expert, a dense product): a patch holds every tile of its row blocks, so that
-// each weight row is fetched into one XCD's L2 only (square patches of 4 x 4 fetched the rows of eight tiles twice).
-inline int patch_all_tiles(int64_t n_rb, int64_t tiles) {
-    if (tiles < 1 || tiles > 16) return patch_edge(n_rb, tiles);
-    int er = 4;
-    while (er > 1 && (n_rb + er - 1) / er < 16) er >>= 1;
-    return er + 256 * (int)tiles;
-}
-inline unsigned patch_grid(int64_t n_rb, int64_t tiles, int patch) {
-    const int er = patch & 255, et = (patch >> 8) ? (patch >> 8) : er;
-    const int64_t RG = (n_rb + er - 1) / er, TG = (tiles + et - 1) / et;
-    return (unsigned)((RG * TG + 7) / 8 * 8 * er * et);
-}
 
 // The combine pass of the layer BEFORE this one, folded into this layer's front kernel (stacks of layers, small batches):
 // the token's input row is  sum of that layer's weighted expert outputs in ascending expert order (+ that layer's

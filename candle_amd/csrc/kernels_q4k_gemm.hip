@@ -41,7 +41,6 @@
 // eight; the minimums leave through the sixteen block sums as for Q4K.
 #include <type_traits>
 #include "act_quant.hpp"
-#include "gemm_plan.hpp"
 #include "kernels.hpp"
 #include "planes.hpp"
 
@@ -566,7 +565,7 @@ static void launch_gemm(ExpertParams& p, hipStream_t s) {
     // lose by it (4096 x 4096 at 1500 rows 90 / 103 and 79 / 92).
     constexpr bool one_operand = MODE == 1 && (FMT == MOE_GGML_Q3K || FMT == MOE_GGML_Q5K || FMT == MOE_GGML_Q6K);
     const bool tiles64 = p.rb.tile_slots == 64;
-    const bool wide = !(one_operand && tiles64) && gemm_wide(MODE == 0, rows, p.n_slots, p.n_groups, p.rb.tile_slots);
+    const bool wide = !(one_operand && tiles64) && gemm_wide(MODE == 0, rows, p.n_slots, p.n_groups, p.rb.tile_slots, tiles);
     const int64_t n_rb = rows / (wide ? 256 : 128);
     p.patch = patch_edge(n_rb, tiles);
     const dim3 grid(patch_grid(n_rb, tiles, p.patch));
