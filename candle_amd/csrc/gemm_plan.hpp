@@ -74,12 +74,14 @@ inline int64_t busiest_xcd(int64_t n_rb, int64_t tiles, int64_t max_tiles) {
 //   1664, 3.12 / 3.25: 282 / 258; 32000 x 4096 at 300, 1.5: 105 / 125; 640, 2.5: 211 / 193; Q6_K 640 238 / 212.
 //   Mixtral shape, us per step: down, 450 tokens, 0.5 rounds 523 / 471; 500 tokens 0.69: 589 / 615; 600 tokens, 1.0: 648 / 667; 1000
 //   tokens, 1.38: 1032 / 984; 2048 tokens, 2.5: 1701 / 1653; up, 301 tokens, 4.0: 375 / 388; 1000 tokens, 9.5 / 8.5: 1030 / 999.
+//   up to 512 rows: always narrow.  One or two wide row blocks leave most of a patch dead, and a CU that is offered a dead wide
+//   workgroup takes nothing else (Q4_K 512 x 4096 at 16384 rows 187 / 138, 256 x 256 at 60000 115 / 68; 768 x 4096 191 / 195).
 //   up projection in tiles of 64 slots: always narrow.  Its lists are short and uneven, and the finer grid shares them out better
 //   (Mixtral shape, 137 / 257 / 287 tokens: Q4_K 280 / 273, 416 / 406, 454 / 433; Q6_K 257 tokens 547 / 521; Q3_K 495 / 470;
 //   200 tokens: Q4_K 318 / 323, Q6_K 479 / 457).
 // rows: weight rows of the launch (w1 and w3 both counted); groups: expert lists, 1 for a dense product; max_tiles: the grid's tiles.
 inline bool gemm_wide(bool up, int64_t rows, int64_t slots, int64_t groups, int tile_slots, int64_t max_tiles) {
-    if (rows % 256 || (up && tile_slots == 64)) return false;
+    if (rows % 256 || rows <= 512 || (up && tile_slots == 64)) return false;
     const int64_t tiles = std::min(gemm_tiles(slots, groups, tile_slots), max_tiles);
     if (rows / 256 * tiles > 12 * 256) return true;   // a tail is less than 5 % of so many rounds
     const int64_t wide = (busiest_xcd(rows / 256, tiles, max_tiles) + 31) / 32;

@@ -68,6 +68,8 @@ def plan(tmp_path_factory):
     (32000, 300, 128, 1),    # 1.5: 105 / 125
     (32000, 512, 128, 1),    # 2.0: 152 / 157
     (32000, 640, 128, 0),    # 2.5: 211 / 193
+    (512, 16384, 128, 0),    # 187 / 138: too few row blocks
+    (768, 16384, 128, 1),    # 191 / 195
     (4224, 1024, 64, 0),     # not a multiple of 256 rows
 ])
 def test_dense_products(plan, n, m, tile, wide):
