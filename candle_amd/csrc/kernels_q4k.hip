@@ -920,8 +920,8 @@ DEF_DOWN_FINE(q6k_down_t2_fine, FmtQ6KP, 2, 4, 4, 2)
 // BlockQ8K::from_float of act_quant.hpp, 64 lanes x 4 elements) into a few hundred bytes of LDS of its own and reads
 // its MFMA operand back from there.  Every workgroup repeats the quantisation of the rows -- ~80 instructions per block
 // and row -- which is why this pays for a handful of rows only: against it stand a kernel launch and a round trip of the
-// quantised rows through memory.  Same blocks, same products, partial sums added in the same order as quantize_rows_kernel
-// followed by the streaming down kernel: the results carry the same bits.
+// quantised rows through memory.  Same blocks, same products, partial sums added in the same order as the row pass
+// (quantize_q8k_rows_kernel) followed by the streaming down kernel: the results carry the same bits.
 constexpr int FUSED_MAX_ROWS = 4;
 constexpr int XQ_BSUM = 256, XQ_D = 288, XQ_BYTES = 320;   // one quantised block in LDS: 256 quants, 16 f16 sums, f32 scale
 constexpr int FUSED_NW = 4;

@@ -19,7 +19,8 @@
 //
 // What bounds it: the issue port of a SIMD, which matrix and vector instructions share (a 16x16x64 MFMA holds it for 8
 // cycles, a vector instruction for 4), with the unpacking (95 vector instructions per 16 rows and super-block) and the
-// results (5 each).  Two weight operands per wave: an LDS read feeds four matrix instructions instead of two.  That
+// results (5 each), and then waiting: counted over the up launch of 4096 tokens at the Mixtral shape the port is taken 75 % of the
+// time, the matrix pipe is busy 50 %, and a wave waits for 30 % of its cycles.  Two weight operands per wave: an LDS read feeds four matrix instructions instead of two.  That
 // takes two waves per SIMD (256 registers), too few to cover each other, so a wave overlaps its own work: the results of
 // operand o - 1 are added up between the matrix instructions of operand o, and the next super-block's transfers are
 // issued a few at a time behind the operands (in one go at the top they held each wave up for 1650 to 4700 of 9000 cycles).
@@ -68,8 +69,6 @@ __device__ __forceinline__ uint32_t scale_bytes(uint32_t q, uint32_t s) {
 
 // A tile is NOP 16-slot MFMA operands: 8 (128 slots) for big batches, 4 (64 slots) when the experts'
 // lists are short, so that less of a tile is padding.
-constexpr int G_WAVES = 8;
-constexpr int G_THREADS = 64 * G_WAVES;
 // Activations in LDS, laid out so that what one MFMA reads is one contiguous stretch in lane order
 // (any other placement of a 16-lane x 4-chunk operand runs into LDS bank conflicts at half the read
 // rate), and so that one direct global->LDS load of a wave (lane i lands at byte 16 i) writes exactly
