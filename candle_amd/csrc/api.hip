@@ -483,19 +483,12 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
     const Switches& sw = switches();
     ForwardPlan pl;
     const bool shared = L->Fs > 0;
-    // K-quant batches with more than 34 rows per expert take the tiled MFMA kernel for the up projection (F a
-    // multiple of 64, H of 128; those kernels address activation rows with 32-bit byte offsets), from ~64 rows per
-    // expert on for the down projection too.  (Mixtral shape, us per step, up streamed / tiled: Q4_K 32 rows per expert 280 / 287,
-    // 34 rows 287 / 295, 35 rows 314 / 276; Q6_K 391 / 389 at 35, 439 / 391 at 38; Q5_K 348 / 378 at 38, 407 / 397 at 43.  Down streamed
-    // / tiled: Q4_K 55 rows 377 / 384, 60 rows 399 / 396, 64 rows 452 / 415; Q5_K 530 / 541 at 64, 529 / 454 at 75; Q6_K tiled from
-    // 35 rows on already, 388 / 361; at a quarter of the width Q4_K streamed at 75 rows still, 57 / 69.)
-    // Their tiles hold 64 slots up to 72 rows per expert, 128 from there.  The line is that of a tiled kernel that
-    // multiplied the dead operands of a tile too; with the present one 128 slots are the better tile from about 60 rows on (Mixtral
-    // shape, 64 / 128 slots: Q4_K 50 rows 324 / 316, 60 rows 390 / 336, 68 rows 433 / 362, 75 rows 444 / 366; Q3_K 55 rows 354 / 366, 60 rows
-    // 446 / 381; a quarter of the width, 68 rows 70 / 68).
-    // (w2 may be Q4K, Q5K or Q6K whatever w1 / w3 are: mixed files store part of it as Q6K)
-    pl.tiled = !sw.no_gemm && q4k_gemm_up_format(L->dt) && L->F % 64 == 0 && L->H % 128 == 0 && T * L->k > 34 * L->E;
-    pl.tiled_down = pl.tiled && q4k_gemm_down_format(L->dt_down) && T * L->k > 64 * L->E;
+    // K-quant batches with more than 34 rows per expert take the tiled MFMA kernels (F a multiple of 64, H of 128; those kernels
+    // address activation rows with 32-bit byte offsets) for the up projection, and for the down projection where gemm_layer_plan
+    // says so.  (Mixtral shape, us per step, up streamed / tiled: Q4_K 32 rows per expert 280 / 287, 34 rows 287 / 295, 35 rows
+    // 314 / 276; Q6_K 391 / 389 at 35, 439 / 391 at 38; Q5_K 348 / 378 at 38, 407 / 397 at 43.)
+    // (w2 may be any K-quant whatever w1 / w3 are: mixed files store part of it as Q6K)
+    pl.tiled = !sw.no_gemm && q4k_gemm_up_format(L->dt) && q4k_gemm_down_format(L->dt_down) && L->F % 64 == 0 && L->H % 128 == 0 && T * L->k > 34 * L->E;
     // 16-slot tiles a workgroup carries per pass over the weights, from the expected rows per expert
     // (a list longer than a pass covers is finished by further workgroups that stream the weights again)
     // (measured at the Mixtral shape: two tiles per pass, with a second pass for the longer lists, beat four
@@ -513,7 +506,12 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
     // lists let an empty pass leave at once; 128 experts, 512 tokens: 386 -> 303 us).
     const int64_t passes = (T + 16 * pl.slot_tiles - 1) / (16 * pl.slot_tiles);
     pl.direct = !pl.tiled && T * L->k <= DIRECT_MAX_SLOTS && T <= DIRECT_MAX_SLOTS && (passes <= 4 || L->E <= 16);
-    pl.tile_slots = sw.tile_slots == 64 || sw.tile_slots == 128 ? sw.tile_slots : T * L->k >= 72 * L->E ? 128 : 64;
+    if (pl.tiled) {
+        const LayerPlan lp = gemm_layer_plan(gemm_format(L->dt), gemm_format(L->dt_down), L->H, L->F, T * L->k, L->E);
+        pl.tile_slots = lp.tile_slots;
+        pl.tiled_down = lp.tiled_down;
+    }
+    if (sw.tile_slots == 64 || sw.tile_slots == 128) pl.tile_slots = sw.tile_slots;
     // Top-2 routing with nothing else to add to a token's result (no shared expert, no residual): the streaming down
     // kernels add their two terms per token straight into the output, which the front kernel clears, and no combine
     // pass runs (a + b is the same float in either order; with three or more terms the order would matter).  Batches
@@ -1219,16 +1217,11 @@ static int enqueue_qlinear(moe_qlinear* Q, const float* d_x, int64_t m, float* d
     // Calls share the quantised rows and the table: a call on another stream waits for the previous one.
     if (!capturing)
         if (int rc = Q->order.enter(s)) return rc;
-    // The tiled MFMA kernel runs one workgroup per (128 or 256 weight rows, tile of 64 or 128 x rows): it pays once that
-    // grid, counted in blocks of 128 rows, fills most of the 256 CUs; below, the streamed kernels split the matrix finer.
-    // (Q4_K, us streamed / tiled: 4096 x 4096 at 256 rows, 128 blocks, 25.0 / 35.2, 320 rows, 160 blocks, 42.5 / 36.0; 1024 x 4096 at 1024
-    // rows, 128 blocks, 30.1 / 40.7, 1400 rows, 176, 48.5 / 41.8; 14336 x 4096 at 128 rows, 224, 42.5 / 47.5, 192 rows, 336, 61.4 / 45.1.
-    // Tiles of 64 / 128 rows: 14336 x 4096 at 256 rows, 224 blocks of the larger tile, 49.6 / 69.4; 32000 x 4096 at 128, 250, 48.8 / 69.3;
-    // 4096 x 4096 at 2048, 512, 96.9 / 83.0.  Between 300 and 512 the larger tile is ahead as well: 4096 x 4096 at 1500, 384, 89.5 / 78.2.)
+    // K-quants: streamed, or tiled with the tile that the costs of gemm_plan.hpp say
     const int64_t row_blocks = Q->n / 128;
-    const int tile_slots = row_blocks * ((m + 127) / 128) >= 512 ? 128 : 64;
-    const bool tiled = !switches().no_gemm && q4k_gemm_down_format(Q->dt) && Q->n % 128 == 0 && m >= 96 &&
-                       row_blocks * ((m + tile_slots - 1) / tile_slots) >= 192;
+    const int k_tile = !switches().no_gemm && q4k_gemm_down_format(Q->dt) ? gemm_dense_tile(gemm_format(Q->dt), Q->n, Q->k, m) : 0;
+    const bool tiled = k_tile != 0;
+    const int tile_slots = tiled ? k_tile : 64;
     // Q8_0 / Q4_0 / Q5_0 matrices: the tiled kernel of the 32-element formats (64-row tiles of the one group, no tile list)
     // once its grid holds a workgroup per CU (Q8_0, 4096 x 4096: 58 against 65 us at 512 rows, 53 against 42 us at 256)
     const bool tiled32 = !switches().no_gemm && q8_0_gemm_usable(Q->dt, 0, Q->n, Q->k) && row_blocks * ((m + 63) / 64) >= 256;

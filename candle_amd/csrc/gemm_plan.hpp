@@ -1,5 +1,5 @@
-// The grids of the tiled kernels: how row blocks and slot tiles are dealt to the XCDs, and how wide the workgroups of a
-// K-quant launch are.  Plain C++: no HIP types.
+// The grids of the tiled kernels: how row blocks and slot tiles are dealt to the XCDs, how wide the workgroups of a K-quant
+// launch are and whether their waves share K, and which slot tile a product takes.  Plain C++: no HIP types.
 #pragma once
 #include <algorithm>
 #include <cstdint>
@@ -88,6 +88,96 @@ inline bool gemm_wide(bool up, int64_t rows, int64_t slots, int64_t groups, int 
     const int64_t narrow = busiest_xcd(rows / 128, tiles, max_tiles), full = narrow / 64, tail = narrow % 64;
     const int64_t halves = 2 * full + (tail == 0 ? 0 : tail <= (full == 1 ? 24 : 32) ? 1 : 2);
     return halves * 21 >= wide * 40;
+}
+
+// What a tiled launch takes, in us, for choosing between its variants.  A workgroup of eight waves (two per SIMD) needs
+//     0.31 us per super-block and 256 weight rows, times (16-slot operands that hold slots + `unpack`),
+// where `unpack` is what the unpacking of a weight costs beside the product with one operand (gemm_unpack below), and 3 us
+// around its K loop; workgroups come in rounds of 32 on the busiest XCD.  Two workgroups of four waves share a CU at 5 % more; one alone
+// takes 0.85 of such a pair's time, which is what makes small grids slow: a wave alone leaves half of its SIMD's cycles
+// empty.  So where a launch would have one of them per CU, the four row groups of a workgroup are given to eight waves, four for
+// each half of K (or two row groups to eight waves, a quarter of K each), and the sums meet in LDS: half (a quarter of) the K
+// steps with every SIMD full, 10 % more per step for the activations fetched per row and 6 us around the loop.
+// Against measurements (Q2_K .. Q6_K, 4096 x 4096, 1024 x 4096, 14336 x 4096 and 4096 x 14336 at 96 to 4096 rows; Mixtral's shape and
+// a quarter of it at 137 to 3000 tokens) the variant chosen by this is 1 % off the best one on average.  One part / the
+// choice: Q4_K 4096 x 4096 at 384 rows 36.8 / 31.6, at 777 51.2 / 45.4, 4096 x 14336 at 512 rows 107 / 90, 14336 x 4096 at 128
+// 47 / 32; Q6_K 4096 x 4096 at 777 58.1 / 49.1; at a full chip it costs: Q4_K 4096 x 4096 at 4096 rows 161 / 181.
+struct GemmPlan {
+    int parts;    // parts K is cut into: 1 (workgroups as gemm_wide says), 2 (128-row workgroups), 4 (64-row ones, tiles of 64 slots)
+    double us;
+};
+// format traits of the tiled kernel: unpack, in operands; one_operand: launches in tiles of 64 slots have one 16-row weight
+// operand per wave; crowded: with 128 slots and the two accumulator sets of a split the registers overflow beyond 96 slots
+struct GemmFormat {
+    double unpack;
+    bool one_operand, crowded;
+    bool four_tiles;   // the streaming kernels carry 64 slots per pass, not 32
+};
+inline GemmPlan gemm_plan(const GemmFormat& f, bool up, int64_t rows, int64_t k, int64_t slots, int64_t groups, int tile_slots, int64_t max_tiles) {
+    const int64_t nsb = k / 256, tiles = std::min(gemm_tiles(slots, groups, tile_slots), max_tiles);
+    // 16-slot operands of a tile: of the longest of a dense product, on average over lists
+    const double ops = groups <= 1 ? (double)std::min<int64_t>(tile_slots / 16, (slots + 15) / 16)
+                                   : std::min((double)tile_slots / 16, (double)gemm_tiles(slots, groups, 16) / (double)std::max<int64_t>(1, tiles));
+    const double step = 0.155 * (f.unpack + ops);   // 128 rows, one super-block
+    auto rounds = [&](int64_t wg_rows) { return (double)((busiest_xcd(rows / wg_rows, tiles, max_tiles) + 31) / 32); };
+    if (rows / 256 * tiles > 12 * 256) return GemmPlan{1, (double)(rows / 256 * tiles) / 256.0 * (2 * step * nsb + 3)};   // a tail hardly counts
+    GemmPlan best{1, 0};
+    const bool one_operand = f.one_operand && !up && tile_slots == 64;
+    if (!one_operand && gemm_wide(up, rows, slots, groups, tile_slots, max_tiles)) {
+        best.us = rounds(256) * (2 * step * nsb + 3);
+    } else {
+        const int64_t n = busiest_xcd(rows / 128, tiles, max_tiles), full = n / 64, tail = n % 64;
+        const double pair = 2.1 * step * nsb + 3, lone = (one_operand ? 1.5 : 1.7) * step * nsb + 3;
+        best.us = full * pair + (tail == 0 ? 0 : tail <= 32 ? lone : pair);
+    }
+    if (up) return best;
+    const double r2 = rounds(128);
+    const double two = r2 * ((r2 > 1 ? 1.2 : 1.1) * (f.crowded && ops > 6 ? 1.5 : 1.0) * step * 2 * (double)((nsb + 1) / 2) + 6);
+    if (two < best.us) best = GemmPlan{2, two};
+    if (tile_slots == 64 && rows % 64 == 0) {
+        const double four = rounds(64) * (0.65 * step * 4 * (double)((nsb + 3) / 4) + 6);
+        if (four < best.us) best = GemmPlan{4, four};
+    }
+    return best;
+}
+// The streaming down kernels, in us.  They give a workgroup 64 rows and a pass of 64 slots (four_tiles: Q4K) in 1.07 us per
+// super-block, in rounds of a workgroup per CU, or passes of 32 slots, where only the number of (16 rows x 32 slots) products
+// counts, 0.83 ns each.
+inline double streamed_us(bool four_tiles, int64_t rows, int64_t k, int64_t slots, int64_t groups) {
+    const int64_t nsb = k / 256, passes = gemm_tiles(slots, groups, four_tiles ? 64 : 32);
+    if (!four_tiles) return 2 + 0.83e-3 * (double)(rows / 16 * passes * nsb);
+    const int64_t wgs = rows / 64 * passes;
+    return 2 + (double)((wgs + 255) / 256 * nsb) * (wgs <= 64 ? 0.7 : 1.07);
+}
+// A routed layer (w1 and w3 of F rows each over H, w2 of H rows over F): the slots per tile, 64 or 128, by the sum of its two
+// launches, and whether the down projection is tiled as well.  (Mixtral shape, us per step, 64 / 128: Q4_K 40 rows per expert
+// 282 / 281, 50 rows 308 / 302, 60 rows 388 / 323, 75 rows 437 / 354; a quarter of its width: 75 rows 60 / 69, 125 rows 76 / 92, 250 rows
+// 126 / 115.  The down launch alone, streamed / tiled: Q4_K 25 rows 69 / 69, 34 rows 99 / 83, 50 rows 112 / 93; Q6_K 34 rows 145 / 105,
+// 50 rows 173 / 118; a quarter of the width Q4_K 35 rows 20 / 17, Q6_K 35 rows 19 / 21, 75 rows 27 / 23.)
+struct LayerPlan {
+    int tile_slots;
+    bool tiled_down;
+};
+inline LayerPlan gemm_layer_plan(const GemmFormat& f_up, const GemmFormat& f_down, int64_t H, int64_t F, int64_t slots, int64_t groups) {
+    const double streamed = streamed_us(f_down.four_tiles, H, F, slots, groups);
+    LayerPlan best{64, false};
+    double us = 0;
+    for (int tile = 64; tile <= 128; tile *= 2) {
+        const int64_t max_tiles = max_gemm_tiles(slots, groups + 1, tile);
+        const double down = gemm_plan(f_down, false, H, F, slots, groups, tile, max_tiles).us;
+        const double t = gemm_plan(f_up, true, 2 * F, H, slots, groups, tile, max_tiles).us + std::min(down, streamed);
+        if (tile == 64 || t <= us) { best = LayerPlan{tile, down <= streamed}; us = t; }
+    }
+    return best;
+}
+// Slots per tile of a dense product of m rows with an [n, k] matrix, or 0 where the streaming kernels are faster.  (us, streamed /
+// tiled: Q4_K 4096 x 4096 at 256 rows 24.9 / 25.0, 320 36 / 31; 1024 x 4096 at 256 18.8 / 23.1, 512 25.6 / 25.3; 14336 x 4096 at
+// 96 38.7 / 29.4; Q6_K 4096 x 4096 at 128 rows 19.7 / 24.4, 192 28.6 / 25.3; 14336 x 4096 at 96 41.4 / 35.8.)
+inline int gemm_dense_tile(const GemmFormat& f, int64_t n, int64_t k, int64_t m) {
+    if (n % 128 || m < 96) return 0;
+    const double us64 = gemm_plan(f, false, n, k, m, 1, 64, max_gemm_tiles(m, 2, 64)).us;
+    const double us128 = gemm_plan(f, false, n, k, m, 1, 128, max_gemm_tiles(m, 2, 128)).us;
+    return streamed_us(f.four_tiles, n, k, m, 1) <= std::min(us64, us128) ? 0 : us128 <= us64 ? 128 : 64;
 }
 
 }  // namespace moe

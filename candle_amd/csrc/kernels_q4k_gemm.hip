@@ -31,6 +31,13 @@
 // (launch_gemm).  Registers: 164 to 254 with two operands (Q5K at 128 slots: 256, one to three of them spilled outside the K
 // loop), 122 to 126 with one.
 //
+// Where a launch would have no more than one workgroup of four waves per CU (a down projection of some hundred tokens, dense products
+// of a few hundred rows), a wave alone on its SIMD leaves it idle for two fifths of the time, and nothing else is there to run.
+// There the workgroup has eight waves for the same rows, four for each half of K with LDS buffers of their own (KS = 2; KS = 4:
+// two waves for each quarter, 64 rows), whose sums meet in LDS at the end.  Down launch, Mixtral shape: Q4_K 200 tokens 112 -> 93 us,
+// 301 tokens 128 -> 111; Q6_K 301 tokens 153 -> 135.  The rule and the dense products' times: gemm_plan.hpp.  On a full chip the split
+// costs (Q4_K 4096 x 4096 at 4096 rows 161 -> 181): there the chip's power is the bound, the clock falls from 2.2 to 1.7 GHz.
+//
 // Q6K weights (the w2 of mixed files) take the same kernel for the down projection.  BlockQ6K::vec_dot
 // (k_quants.rs:1613-1671) is d * y.d * sum_j sc_j * ((code_j - 32) . q8_j) with an i8 scale per 16 elements; the
 // products W = sc * (code - 32) (|W| <= 4096) are formed in packed 16-bit arithmetic and cut into two signed bytes,
@@ -433,20 +440,25 @@ __device__ __forceinline__ float silu_gemm(float v) { return v / (1.0f + __expf(
 // J 16-row weight operands per wave, NW waves per workgroup, 4 / J waves per SIMD; a tile of NOP*16 slots.
 // MODE 0: up   -- a wave carries 16 rows of w1 and the same 16 rows of w3 (J = 2) and writes h = silu(a) * b (f32).
 // MODE 1: down -- 16 J rows of w2 per wave; writes yw.
-// FMT: the weights' format (Q2K ... Q6K).
-template <int FMT, int MODE, int NOP, int NW, int J>
+// FMT: the weights' format (Q2K ... Q6K).  KS: parts the waves of a workgroup cut K into.
+template <int FMT, int MODE, int NOP, int NW, int J, int KS = 1>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4 / J, 4 / J))) void q4k_gemm_kernel(ExpertParams p) {
     static_assert(J == 2 || (J == 1 && MODE == 1), "the up projection takes w1 and w3 side by side");
+    static_assert(KS == 1 || (MODE == 1 && NW % KS == 0 && NOP % KS == 0), "the up projection's waves walk all of K");
     static_assert(FMT == MOE_GGML_Q2K || FMT == MOE_GGML_Q3K || FMT == MOE_GGML_Q4K || FMT == MOE_GGML_Q5K || FMT == MOE_GGML_Q6K, "formats of the tiled kernel");
-    constexpr int NB = NOP * 4 / NW;
+    constexpr int NWR = NW / KS;    // waves that share a part of K, each with rows of its own
+    constexpr int NB = NOP * 4 / NWR;
+    static_assert(NOP / 2 <= NWR, "one transfer of block sums per wave");
     constexpr int TILE_BYTES = FMT == MOE_GGML_Q6K ? Q6K_TILE_BYTES : FMT == MOE_GGML_Q5K ? Q5K_TILE_BYTES : FMT == MOE_GGML_Q2K ? Q2K_TILE_BYTES : FMT == MOE_GGML_Q3K ? Q3K_TILE_BYTES : Q4K_TILE_BYTES;
     constexpr bool kSums = FMT != MOE_GGML_Q6K && FMT != MOE_GGML_Q3K;   // block sums staged (the mins term)
-    __shared__ GemmLds<NOP> L;
+    __shared__ GemmLds<NOP> L_all[KS];
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KS == 1 ? wave_id : wave_id % NWR, kpart = KS == 1 ? 0 : wave_id / NWR;
+    GemmLds<NOP>& L = L_all[kpart];
     const int n_tiles = p.rb.tile_tab[0];
     // workgroup -> (row block, slot tile), in patches per XCD (patch_position)
-    const int n_rb = MODE == 0 ? p.F / (16 * NW) : p.H / (16 * J * NW);
+    const int n_rb = MODE == 0 ? p.F / (16 * NW) : p.H / (16 * J * NWR);
     const PatchPos pos = patch_position((int)blockIdx.x, n_rb, p.patch);
     const int rblk = pos.rblk, tile = pos.tile;
     if (tile >= n_tiles || rblk >= n_rb) return;
@@ -474,7 +486,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4 / J, 
 
     // weight operands of this wave
     const GroupWeights gw = p.groups[grp];
-    const int row0 = (rblk * NW + wave) * (MODE == 0 ? 16 : 16 * J);
+    const int row0 = (rblk * NWR + wave) * (MODE == 0 ? 16 : 16 * J);
     const uint8_t* wp[J];
     if (MODE == 0) {
         wp[0] = gw.w1 + (size_t)(row0 / 16) * TILE_BYTES;
@@ -491,40 +503,46 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4 / J, 
 
     // operands of the tile that hold slots of the list: a short tile's others are neither fetched nor multiplied
     const int live = __builtin_amdgcn_readfirstlane(min(NOP, (n_g - pos0 + 15) >> 4));
+    // the super-blocks of this wave's part of K
+    const int sb_lo = KS == 1 ? 0 : kpart * (nsb / KS) + min(kpart, nsb % KS), n_sb = KS == 1 ? nsb : nsb / KS + (kpart < nsb % KS ? 1 : 0);
+    const int n_steps = (nsb + KS - 1) / KS;
+    const int sb_first = KS == 1 ? 0 : min(sb_lo, nsb - 1);   // (fewer super-blocks than parts: requested, never multiplied)
     auto stage = [&](auto I, int sb, int buf) { stage_piece<decltype(I)::value, kSums, NOP, NB>(ab, rows, sb, L, buf, wave, live); };
-    static_for<0, NB + 2>([&](auto I) { stage(I, 0, 0); });
+    static_for<0, NB + 2>([&](auto I) { stage(I, sb_first, 0); });
     BRegs raw[J];
 #pragma unroll
-    for (int j = 0; j < J; j++) raw[j] = b_load<FMT>(wp[j], lane);
+    for (int j = 0; j < J; j++) raw[j] = b_load<FMT>(wp[j] + (size_t)sb_first * sb_stride, lane);
     wait_all_loads();
     __syncthreads();
     // the K loop over LV operands
     auto run = [&](auto lv_tag) {
         constexpr int LV = decltype(lv_tag)::value;
-        for (int sb = 0; sb < nsb; sb++) {
-            const int buf = sb & 1, nb = buf ^ 1;
-            const int sbn = sb + 1 < nsb ? sb + 1 : sb;
-            BPlanes B[J];
+        for (int it = 0; it < n_steps; it++) {
+            const int buf = it & 1, nb = buf ^ 1;
+            const int sb = sb_lo + it, sbn = it + 1 < n_sb ? sb + 1 : sb;
+            if (KS == 1 || it < n_sb) {   // (wave-uniform: a part may be one super-block shorter)
+                BPlanes B[J];
 #pragma unroll
-            for (int j = 0; j < J; j++) B[j] = b_planes<FMT>(raw[j], lane);
-            // (for the sake of the registers the next weights are requested after this super-block's are unpacked)
-            __builtin_amdgcn_sched_barrier(0);
-            v4i a[4];
+                for (int j = 0; j < J; j++) B[j] = b_planes<FMT>(raw[j], lane);
+                // (for the sake of the registers the next weights are requested after this super-block's are unpacked)
+                __builtin_amdgcn_sched_barrier(0);
+                v4i a[4];
 #pragma unroll
-            for (int P = 0; P < 4; P++) a[P] = operand_piece(L.q[buf], 0, P, lane);
-            OperandAcc<J> prev;
-            // The next super-block's weights and activations are requested while the operands are multiplied, a few requests at a
-            // time: issued in one go they fill the CU's memory queue and the wave stands still for a thousand cycles and more.
-            gemm_operands<FMT, NOP, LV, 0, J>(B, L, buf, lane, a, prev, facc, [&](auto o_tag) {
-                constexpr int O = decltype(o_tag)::value;
-                // (four waves per SIMD: a format with block sums has registers for the next weights behind its last operand only)
-                if constexpr (O == (J == 1 && kSums ? LV - 1 : 0)) raw[0] = b_load<FMT>(wp[0] + (size_t)sbn * sb_stride, lane);
-                if constexpr (J == 2 && O == (LV > 2 ? 1 : 0)) raw[J - 1] = b_load<FMT>(wp[J - 1] + (size_t)sbn * sb_stride, lane);
-                constexpr int FIRST = LV > 2 ? 1 : 0, SPAN = LV > 4 ? LV - 3 : 1;
-                static_for<0, NB + 2>([&](auto I) {
-                    if constexpr (FIRST + decltype(I)::value * SPAN / (NB + 2) == O) stage(I, sbn, nb);
+                for (int P = 0; P < 4; P++) a[P] = operand_piece(L.q[buf], 0, P, lane);
+                OperandAcc<J> prev;
+                // The next super-block's weights and activations are requested while the operands are multiplied, a few requests at a
+                // time: issued in one go they fill the CU's memory queue and the wave stands still for a thousand cycles and more.
+                gemm_operands<FMT, NOP, LV, 0, J>(B, L, buf, lane, a, prev, facc, [&](auto o_tag) {
+                    constexpr int O = decltype(o_tag)::value;
+                    // (four waves per SIMD: a format with block sums has registers for the next weights behind its last operand only)
+                    if constexpr (O == (J == 1 && kSums ? LV - 1 : 0)) raw[0] = b_load<FMT>(wp[0] + (size_t)sbn * sb_stride, lane);
+                    if constexpr (J == 2 && O == (LV > 2 ? 1 : 0)) raw[J - 1] = b_load<FMT>(wp[J - 1] + (size_t)sbn * sb_stride, lane);
+                    constexpr int FIRST = LV > 2 ? 1 : 0, SPAN = LV > 4 ? LV - 3 : 1;
+                    static_for<0, NB + 2>([&](auto I) {
+                        if constexpr (FIRST + decltype(I)::value * SPAN / (NB + 2) == O) stage(I, sbn, nb);
+                    });
                 });
-            });
+            }
             wait_all_loads();
             __syncthreads();
         }
@@ -536,6 +554,41 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4 / J, 
 
     // epilogue: lane holds weight row n = lane%16 of its operands and slots 16 o + 4 (lane/16) + i
     const int n = lane & 15, g = lane >> 4;
+    if constexpr (KS > 1) {
+        // the parts' sums meet in LDS (the loop's last barrier has released it); the waves of part q add up, in the order of the
+        // parts, and store operands q NOP / KS ...
+        float* xch = reinterpret_cast<float*>(L_all);   // [wave][operand][j][i][lane]
+        static_assert(NW * NOP * J * 4 * 64 * sizeof(float) <= sizeof(L_all), "exchange area");
+#pragma unroll
+        for (int o = 0; o < NOP; o++)
+#pragma unroll
+            for (int j = 0; j < J; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) xch[(((wave_id * NOP + o) * J + j) * 4 + i) * 64 + lane] = facc[o][j][i];
+        __syncthreads();
+#pragma unroll
+        for (int oo = 0; oo < NOP / KS; oo++) {
+            const int o = kpart * (NOP / KS) + oo;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int pos = pos0 + o * 16 + g * 4 + i;
+                if (pos >= n_g) continue;
+                const int slot = s_begin + pos;
+                const float w = p.rb.perm_w[slot];
+#pragma unroll
+                for (int j = 0; j < J; j++) {
+                    float sum = 0.f;
+#pragma unroll
+                    for (int q = 0; q < KS; q++) {
+                        const float part = xch[((((q * NWR + wave) * NOP + o) * J + j) * 4 + i) * 64 + lane];
+                        sum = q == 0 ? part : sum + part;
+                    }
+                    p.yw[(int64_t)slot * p.H + row0 + 16 * j + n] = sum * w;
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int o = 0; o < NOP; o++)
 #pragma unroll
@@ -564,20 +617,28 @@ static void launch_gemm(ExpertParams& p, hipStream_t s) {
     // lose by it (4096 x 4096 at 1500 rows 90 / 103 and 79 / 92).
     constexpr bool one_operand = MODE == 1 && (FMT == MOE_GGML_Q3K || FMT == MOE_GGML_Q5K || FMT == MOE_GGML_Q6K);
     const bool tiles64 = p.rb.tile_slots == 64;
+    auto launch = [&](auto kernel, int waves, int64_t wg_rows) {
+        const int64_t n_rb = rows / wg_rows;
+        p.patch = patch_edge(n_rb, tiles);
+        hipLaunchKernelGGL(kernel, dim3(patch_grid(n_rb, tiles, p.patch)), dim3(waves * 64), 0, s, p);
+    };
+    // K split over the waves of a workgroup where the grid would leave SIMDs with one wave or none (gemm_plan)
+    if constexpr (MODE == 1) {
+        const int parts = gemm_plan(gemm_format(FMT), false, rows, p.F, p.n_slots, p.n_groups, p.rb.tile_slots, tiles).parts;
+        if (parts == 4) return launch(q4k_gemm_kernel<FMT, 1, 4, 8, 2, 4>, 8, 64);
+        if (parts == 2) return tiles64 ? launch(q4k_gemm_kernel<FMT, 1, 4, 8, 2, 2>, 8, 128) : launch(q4k_gemm_kernel<FMT, 1, 8, 8, 2, 2>, 8, 128);
+    }
     const bool wide = !(one_operand && tiles64) && gemm_wide(MODE == 0, rows, p.n_slots, p.n_groups, p.rb.tile_slots, tiles);
-    const int64_t n_rb = rows / (wide ? 256 : 128);
-    p.patch = patch_edge(n_rb, tiles);
-    const dim3 grid(patch_grid(n_rb, tiles, p.patch));
     if (!tiles64) {
-        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 8, 2>), grid, dim3(512), 0, s, p);
-        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 8, 4, 2>), grid, dim3(256), 0, s, p);
+        if (wide) launch(q4k_gemm_kernel<FMT, MODE, 8, 8, 2>, 8, 256);
+        else launch(q4k_gemm_kernel<FMT, MODE, 8, 4, 2>, 4, 128);
     } else if constexpr (one_operand) {
-        hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8, 1>), grid, dim3(512), 0, s, p);
+        launch(q4k_gemm_kernel<FMT, MODE, 4, 8, 1>, 8, 128);
     } else if constexpr (MODE == 0) {
-        hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4, 2>), grid, dim3(256), 0, s, p);
+        launch(q4k_gemm_kernel<FMT, MODE, 4, 4, 2>, 4, 128);
     } else {
-        if (wide) hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 8, 2>), grid, dim3(512), 0, s, p);
-        else hipLaunchKernelGGL((q4k_gemm_kernel<FMT, MODE, 4, 4, 2>), grid, dim3(256), 0, s, p);
+        if (wide) launch(q4k_gemm_kernel<FMT, MODE, 4, 8, 2>, 8, 256);
+        else launch(q4k_gemm_kernel<FMT, MODE, 4, 4, 2>, 4, 128);
     }
 }
 bool q4k_gemm_up_format(int dt) { return dt == MOE_GGML_Q2K || dt == MOE_GGML_Q3K || dt == MOE_GGML_Q4K || dt == MOE_GGML_Q5K || dt == MOE_GGML_Q6K; }
