@@ -523,6 +523,21 @@ __device__ __forceinline__ void q32s_engine(const uint8_t* const tp[NT], size_t 
     }
 }
 
+// Maximum / sum over the 32 lanes that hold one block, left in all of them: four rotations inside the rows of 16 lanes
+// (DPP: no LDS traffic, no address arithmetic) and one exchange between the two rows.
+__device__ __forceinline__ float block32_max(float v) {
+#define GV_ROR_MAX(n) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + (n), 0xf, 0xf, false)))
+    GV_ROR_MAX(8); GV_ROR_MAX(4); GV_ROR_MAX(2); GV_ROR_MAX(1);
+#undef GV_ROR_MAX
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401f)));   // lane ^ 16
+}
+__device__ __forceinline__ int block32_sum(int v) {
+#define GV_ROR_ADD(n) v += __builtin_amdgcn_update_dpp(0, v, 0x120 + (n), 0xf, 0xf, false)
+    GV_ROR_ADD(8); GV_ROR_ADD(4); GV_ROR_ADD(2); GV_ROR_ADD(1);
+#undef GV_ROR_ADD
+    return v + __builtin_amdgcn_ds_swizzle(v, 0x401f);
+}
+
 // (a fixed number of waves per SIMD also makes the compiler keep the MFMA results in ordinary registers)
 template <int DT, int TT, bool ONCE, int WPE, int DEPTH>
 __global__ __launch_bounds__(Q32_THREADS) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void q32s_up_kernel(ExpertParams p) {
@@ -640,6 +655,223 @@ __global__ __launch_bounds__(Q32_THREADS) __attribute__((amdgpu_waves_per_eu(WPE
         }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The two streaming kernels again for launches of few workgroups (a small layer, a handful of tokens, dense matrices of a few
+// thousand rows): workgroups of a quarter of the rows, so that four times as many of them fill the chip.  Same arithmetic, same
+// order of additions.
+//
+// Up: a workgroup owns 32 rows of F -- one block of h per slot -- and its four waves one 16-row tile of w1 or w3 each, all of
+// K.  The sums meet in LDS, where every wave evaluates silu for a quarter of them and the blocks are quantised.
+//   1024 -> 3584, eight experts, 16 tokens, Q4_0: 224 workgroups, one wave per SIMD, 16.7 us -> 896 workgroups 14.5.  What is left is
+//   latency: the slot list, the first loads, eight barriers, silu and the quantisation.
+template <int DT, int DEPTH>
+__global__ __launch_bounds__(Q32_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void q32s_up_fine_kernel(ExpertParams p) {
+    __shared__ int list_lds[DIRECT_MAX_SLOTS];
+    __shared__ int wtot_lds[Q32_THREADS / 64];
+    __shared__ __align__(16) uint8_t act_lds[2 * Q32S_ACT_BYTES];
+    __shared__ float xch[4][2][64];     // [wave][result it leaves to its partner][lane]
+    __shared__ float hx[16][33];        // h: [slot][row]
+    __shared__ uint64_t exp_tab[32];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    if (tid < 32) exp_tab[tid] = exp2f_tab(tid);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = __builtin_amdgcn_readfirstlane(group_of_row(p, blockIdx.y));
+    if (grp < 0) return;
+    const GroupSlots gs = group_slots<Q32_THREADS>(p, grp, list_lds, wtot_lds);
+    const int tg0 = blockIdx.z * 16;
+    if (tg0 >= gs.n) return;
+    const int H = p.H, F = p.F, n_rt = F / 16, fb = blockIdx.x;
+    constexpr size_t STB = Q32SFmt<DT>::STB;
+    Q32SRows<1> st;
+    {
+        const int iq = tg0 + (tid >> 4), is = tg0 + ((tid >> 2) & 15);
+        st.q_row[0] = (uint32_t)slot_token(p, gs.slot(iq < gs.n ? iq : gs.n - 1));
+        st.s_row[0] = (uint32_t)slot_token(p, gs.slot(is < gs.n ? is : gs.n - 1));
+    }
+    const GroupWeights gw = p.groups[grp];
+    // waves 0, 1: the block's two tiles of w1; 2, 3: of w3
+    const uint8_t* tp[1] = {(wave < 2 ? gw.w1 : gw.w3) + (size_t)(2 * fb + (wave & 1)) * STB};
+    float acc[1][1][4] = {{{0.f, 0.f, 0.f, 0.f}}};
+    q32s_engine<DT, 1, 1, true, DEPTH>(tp, (size_t)n_rt * STB, p.xq, H, st, act_lds, tid, acc);
+    // h = silu(w1 x) * (w3 x): the w1 wave takes results 0 and 1, the w3 wave results 2 and 3 of their rows
+#pragma unroll
+    for (int i = 0; i < 2; i++) xch[wave][i][lane] = wave < 2 ? acc[0][0][2 + i] : acc[0][0][i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float other = xch[wave ^ 2][i][lane];
+        const float gate_v = wave < 2 ? acc[0][0][i] : other, up_v = wave < 2 ? other : acc[0][0][2 + i];
+        hx[4 * g + (wave < 2 ? 0 : 2) + i][(wave & 1) * 16 + r] = silu_ref32(gate_v, exp_tab) * up_v;
+    }
+    __syncthreads();
+    // half a wave quantises a slot's block
+    const int nfb = F / 32, e = lane & 31;
+#pragma unroll
+    for (int it = 0; it < 2; it++) {
+        const int s16 = it * 8 + (tid >> 5);
+        const float x = hx[s16][e];
+        const float amax = block32_max(fabsf(x));
+        const float d = amax / 127.0f;
+        const float id = (d != 0.f) ? 1.0f / d : 0.f;
+        const int q = round_as_i8(x * id);
+        const int sum = block32_sum(q);
+        if (tg0 + s16 < gs.n) {
+            const int64_t hrow = gs.slot(tg0 + s16) - p.slot_origin;
+            p.hq.qs[hrow * F + fb * 32 + e] = (int8_t)q;
+            if (e == 0) {
+                const float dh = __half2float(__float2half_rn(d));
+                p.hq.d[hrow * nfb + fb] = dh;
+                reinterpret_cast<int32_t*>(p.hq.bsum)[hrow * nfb + fb] = q8_block_word(vecdot_dtype(DT), sum, dh);
+            }
+        }
+    }
+}
+
+// Down: a workgroup owns one 16-row tile and its four waves take the K steps (128 elements, four blocks) in turn.  They park the block
+// values ((isum as f32) * d_w) * d_x (+ m_w * s_x) in LDS, sixteen blocks a round, and then every thread adds its result's sixteen
+// in block order.  A wave stages its own step's activations (no barrier but the round's).
+//   3584 -> 1024, eight experts, 16 tokens, Q4_0: 128 workgroups, a wave per tile walking 112 blocks and 28 barriers, 19.8 us ->
+//   512 workgroups, four per CU, 12.3.  (Two buffers of block values would save a barrier a round but leave three workgroups per CU:
+//   4096 x 4096, Q8_0, 64 rows 22.5 us against 18.6.)
+constexpr int Q32F_BLK = 640;                          // LDS bytes of one block's operand, 512 padded: a wave writes four blocks at once
+constexpr int Q32F_ACT = 4 * Q32F_BLK + 2 * 4 * 16 * 4;   // ... of a step: operands, then scales and words [block][slot]
+template <int DT, int DEPTH>
+__global__ __launch_bounds__(Q32_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void q32s_down_fine_kernel(ExpertParams p) {
+    typedef Q32Fmt<DT> F32;
+    constexpr bool WORDS = F32::OFFSET != 0 || F32::HAS_M;
+    __shared__ int list_lds[DIRECT_MAX_SLOTS];
+    __shared__ int wtot_lds[Q32_THREADS / 64];
+    __shared__ float terms[16][256];                   // [block of the round][result i * 64 + lane]
+    __shared__ __align__(16) uint8_t act[4][Q32F_ACT];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = __builtin_amdgcn_readfirstlane(group_of_row(p, blockIdx.y)), rt = blockIdx.x;
+    if (grp < 0) return;
+    const int H = p.H, K = p.F, nkb = K / 32, nks = K / 128, n_rt = H / 16;
+    const int n_rounds = (nks + 3) / 4;
+    constexpr size_t STB = Q32SFmt<DT>::STB;
+    const size_t stride = (size_t)n_rt * STB;
+    if (blockIdx.z > 0 && !p.rb.direct && !p.is_shared) {   // a later pass over a measured list: its length before anything is requested
+        const int gi = p.group0 + grp;
+        if ((int)blockIdx.z * 16 >= p.rb.offsets[gi + 1] - p.rb.offsets[gi]) return;
+    }
+    const uint8_t* tp = p.groups[grp].w2 + (size_t)rt * STB;
+    auto step_of = [&](int round) {   // (past the end: the last step again, its values are not added)
+        const int ks = 4 * round + wave;
+        return ks < nks ? ks : nks - 1;
+    };
+    Q32SRaw<DT> ring[DEPTH];
+#pragma unroll
+    for (int j = 0; j < DEPTH; j++) ring[j] = load_q32s<DT, true>(tp + (size_t)step_of(j) * stride, lane);
+    const GroupSlots gs = group_slots<Q32_THREADS>(p, grp, list_lds, wtot_lds);
+    const int tg0 = blockIdx.z * 16;
+    if (tg0 >= gs.n) return;
+    // the lane copies block lane % 4 of slot lane / 4
+    const int ls = lane >> 2, lb = lane & 3;
+    const uint32_t row = (uint32_t)(gs.slot(tg0 + ls < gs.n ? tg0 + ls : gs.n - 1) - p.slot_origin);
+    u32x4g q_lo[DEPTH], q_hi[DEPTH];
+    float dd[DEPTH];
+    int ww[DEPTH];
+    auto request = [&](int j, int round) {
+        const int ks = step_of(round);
+        const uint32_t off = row * (uint32_t)K + (uint32_t)(ks * 128 + lb * 32);
+        q_lo[j] = ldg<u32x4g>(p.hq.qs, off);
+        q_hi[j] = ldg<u32x4g>(p.hq.qs, off + 16);
+        const uint32_t so = (row * (uint32_t)nkb + (uint32_t)(ks * 4 + lb)) * 4u;
+        dd[j] = ldg<float>(p.hq.d, so);
+        if (WORDS) ww[j] = ldg<int>(p.hq.bsum, so);
+    };
+#pragma unroll
+    for (int j = 0; j < DEPTH; j++) request(j, j);
+    uint8_t* mine = act[wave];
+    float* sc = reinterpret_cast<float*>(mine + 4 * Q32F_BLK);
+    int* wd = reinterpret_cast<int*>(mine + 4 * Q32F_BLK + 256);
+    float acc = 0.f;
+    for (int r0 = 0; r0 < n_rounds; r0 += DEPTH) {
+#pragma unroll
+        for (int j = 0; j < DEPTH; j++) {
+            const int round = r0 + j;
+            if (round < n_rounds) {   // uniform over the workgroup
+                // elements 4g .. 4g+3 and 16+4g .. of the block to lane (slot, g)'s eight bytes
+#pragma unroll
+                for (int gg = 0; gg < 4; gg++) {
+                    const u32x2g v = {q_lo[j][gg], q_hi[j][gg]};
+                    *reinterpret_cast<u32x2g*>(mine + lb * Q32F_BLK + (gg * 16 + ls) * 8) = v;
+                }
+                sc[lb * 16 + ls] = dd[j];
+                if (WORDS) wd[lb * 16 + ls] = F32::OFFSET ? Q32S_MAGIC_BITS - ww[j] * F32::OFFSET : ww[j];
+                const Q32SRaw<DT> cur = ring[j];
+                request(j, round + DEPTH);
+                ring[j] = load_q32s<DT, true>(tp + (size_t)step_of(round + DEPTH) * stride, lane);
+                // the wave reads what its other lanes have written: LDS serves a wave's requests in order
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const Q32Tile<DT> wb[4] = {q32s_block<DT, 0>(cur, g), q32s_block<DT, 1>(cur, g), q32s_block<DT, 2>(cur, g), q32s_block<DT, 3>(cur, g)};
+                float (*out)[256] = &terms[wave * 4];
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const uint2 a = *reinterpret_cast<const uint2*>(mine + b * Q32F_BLK + lane * 8);
+                    const f32x4g yd = *reinterpret_cast<const f32x4g*>(sc + b * 16 + 4 * g);
+                    v4i w4 = {0, 0, 0, 0};
+                    if (WORDS) w4 = *reinterpret_cast<const v4i*>(wd + b * 16 + 4 * g);
+                    float t[4] = {0.f, 0.f, 0.f, 0.f};
+                    q32s_mac<DT>(wb[b], a, yd, w4, t);   // 0 + the block's value
+#pragma unroll
+                    for (int i = 0; i < 4; i++) out[b][i * 64 + lane] = t[i];
+                }
+                __syncthreads();
+                const int nb = nkb - 16 * round < 16 ? nkb - 16 * round : 16;
+                const float* in = &terms[0][tid];
+                if (nb == 16) {
+                    float t[16];
+#pragma unroll
+                    for (int b = 0; b < 16; b++) t[b] = in[b * 256];
+#pragma unroll
+                    for (int b = 0; b < 16; b++) acc += t[b];
+                } else {
+                    for (int b = 0; b < nb; b++) acc += in[b * 256];
+                }
+                __syncthreads();   // the next round's values go to the same place
+            }
+        }
+    }
+    // the thread's result: weight row r, slot 4 g + wave
+    const int pos = tg0 + 4 * g + wave;
+    if (pos < gs.n) {
+        const int slot = gs.slot(pos);
+        emit_expert_output(p, slot, rt * 16 + r, acc * slot_weight(p, slot));
+    }
+}
+
+// When the fine kernels are the faster ones.  Counted in workgroups of the coarse kernels (128 rows of F, 64 of H) over passes of 16
+// slots that find slots: up to 700 for the up projection, a list's second and later passes counted twice (they read its
+// weights again); up to 400 for the down projection.  Up, us, coarse / fine: a quarter of Mixtral's width, Q4_0, 224 (up to 40 tokens)
+// 16.8 / 14.6, 448 (100 tokens, two passes) 31.4 / 28.0, three passes 32.8 / 37.2; Qwen-MoE shape, Q8_0, 44 (one token) 31 / 15, 176
+// 47 / 21, 660 (16 tokens) 54 / 43, (64 tokens) 67 / 63; Mixtral, Q4_0, 448 (two tokens) 85 / 56, 896 93 / 97.  Down: a quarter of Mixtral's width
+// 32 17.8 / 10.0, 128 19.8 / 12.3, 256 27.3 / 22.7; Mixtral 128 55 / 32, 256 63 / 51, 512 64 / 81; Qwen-MoE shape 256 14.3 / 12.0, 512 18.6 / 18.8;
+// dense Q8_0 4096 x 4096 64 (16 rows) 21.4 / 11.4, 256 27.8 / 18.6, 448 28.4 / 27.7, 512 28.9 / 30.8; 4096 x 14336 320 84 / 77, 448 87 / 95.
+// A one-tile launch some of whose lists may need a second pass stays coarse in the up projection (Q4_0, 64 tokens 20.8 / 22.6).
+struct Q32Passes {
+    int64_t all, first;   // passes that find slots, and those among them that are their list's first
+};
+static Q32Passes q32_passes(const ExpertParams& p) {
+    if (p.n_groups == 1) return Q32Passes{(p.max_rows + 15) / 16, 1};
+    const int64_t slots = (int64_t)p.rb.T * p.rb.k, first = std::min<int64_t>(p.n_groups, slots);
+    return Q32Passes{std::max(gemm_tiles(slots, p.n_groups, 16), first), first};   // (lists as evenly filled as gemm_tiles takes them)
+}
+static bool q32_up_fine(const ExpertParams& p, int slot_tiles) {
+    const Q32Passes n = q32_passes(p);
+    return (p.F / 32 + 3) / 4 * (2 * n.all - n.first) <= 700 && (slot_tiles > 1 || n.all == n.first);
+}
+static bool q32_down_fine(const ExpertParams& p) { return (p.H / 16 + 3) / 4 * q32_passes(p).all <= 400; }
+// The grid of a fine launch: a row of workgroups per assignment where there are fewer of them than experts.
+static dim3 q32_fine_grid(ExpertParams& p, int64_t row_blocks) {
+    const int64_t slots = (int64_t)p.rb.T * p.rb.k;
+    p.by_assignment = p.rb.direct && !p.is_shared && slots < p.n_groups ? 1 : 0;
+    return dim3((unsigned)row_blocks, (unsigned)(p.by_assignment ? slots : p.n_groups), (unsigned)((p.max_rows + 15) / 16));
+}
+
 template <int DT, int TT>
 static void launch_q32s_up(const ExpertParams& p, dim3 grid, hipStream_t s) {
     // waves per SIMD the register count of each variant allows (the five-bit formats carry their fifth-bit words)
@@ -656,6 +888,12 @@ static hipError_t launch_q32_up_t(const ExpertParams& p, hipStream_t s) {
     const int wpb = Q32_THREADS / 64;
     const int n_pairs = p.F / 32;
     dim3 grid((unsigned)((n_pairs + wpb - 1) / wpb), (unsigned)p.n_groups, (unsigned)((p.max_rows + tt * 16 - 1) / (tt * 16)));
+    if (stream && q32_up_fine(p, tt)) {
+        ExpertParams q = p;
+        const dim3 fine = q32_fine_grid(q, n_pairs);
+        hipLaunchKernelGGL((q32s_up_fine_kernel<DT, 2>), fine, dim3(Q32_THREADS), 0, s, q);
+        return hipGetLastError();
+    }
     if (stream) {
         if (tt == 1) launch_q32s_up<DT, 1>(p, grid, s);
         else launch_q32s_up<DT, 2>(p, grid, s);
@@ -685,6 +923,12 @@ static hipError_t launch_q32_down_t(const ExpertParams& p, hipStream_t s) {
     const int tt = p.slot_tiles >= 2 ? 2 : 1;
     const int wpb = Q32_THREADS / 64;
     dim3 grid((unsigned)((p.H / 16 + wpb - 1) / wpb), (unsigned)p.n_groups, (unsigned)((p.max_rows + tt * 16 - 1) / (tt * 16)));
+    if (stream && q32_down_fine(p)) {
+        ExpertParams q = p;
+        const dim3 fine = q32_fine_grid(q, p.H / 16);
+        hipLaunchKernelGGL((q32s_down_fine_kernel<DT, 2>), fine, dim3(Q32_THREADS), 0, s, q);
+        return hipGetLastError();
+    }
     if (stream) {
         if (tt == 1) launch_q32s_down<DT, 1>(p, grid, s);
         else launch_q32s_down<DT, 2>(p, grid, s);
@@ -987,21 +1231,6 @@ hipError_t launch_q8_0_gemm_down(const ExpertParams& p_in, hipStream_t s) {
 // (+ m_w * s_x) in parallel, 64 blocks at a time, and park them in LDS; one wave then adds them to the running sums in
 // block order.  The rows are quantised inside the kernel (BlockQ8_0 / BlockQ8_1::from_float, k_quants.rs:605-634, 700-729:
 // the arithmetic of quantize_q8_0_block, eight pairs of blocks side by side), each wave the blocks it multiplies.
-// Maximum / sum over the 32 lanes that hold one block, left in all of them: four rotations inside the rows of 16 lanes
-// (DPP: no LDS traffic, no address arithmetic) and one exchange between the two rows.
-__device__ __forceinline__ float block32_max(float v) {
-#define GV_ROR_MAX(n) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + (n), 0xf, 0xf, false)))
-    GV_ROR_MAX(8); GV_ROR_MAX(4); GV_ROR_MAX(2); GV_ROR_MAX(1);
-#undef GV_ROR_MAX
-    return fmaxf(v, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401f)));   // lane ^ 16
-}
-__device__ __forceinline__ int block32_sum(int v) {
-#define GV_ROR_ADD(n) v += __builtin_amdgcn_update_dpp(0, v, 0x120 + (n), 0xf, 0xf, false)
-    GV_ROR_ADD(8); GV_ROR_ADD(4); GV_ROR_ADD(2); GV_ROR_ADD(1);
-#undef GV_ROR_ADD
-    return v + __builtin_amdgcn_ds_swizzle(v, 0x401f);
-}
-
 constexpr int GV_MAX_ROWS = 4;
 constexpr int GV_STEPS = 4;                     // K steps (of four blocks) a wave takes per chunk
 constexpr int GV_BLOCKS = 4 * GV_STEPS;         // blocks per wave and chunk
