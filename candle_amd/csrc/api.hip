@@ -496,8 +496,10 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
     // (the 32-element kernels carry at most two tiles: three or four per pass measured slower at the Mixtral shape and
     // 8 % faster at best where sixty small experts' weights exceed the caches)
     // (K-quants, Mixtral shape: one tile with a second pass for the lists beyond 16 rows beats two tiles up to ~13 rows per
-    // expert on average: 48 tokens 168 against 181 us per step, 64 tokens 214 against 185)
-    const int64_t two_from = (L->vdt == MOE_GGML_Q8K ? 13 : 9) * L->E;
+    // expert on average: 48 tokens 168 against 181 us per step, 64 tokens 214 against 185.  32-element formats: up to 16 rows:
+    // Mixtral shape, Q4_0, 10 rows 175 against 273, 16 rows 258 against 277, 20 rows 294 against 277; Qwen-MoE shape, Q8_0, 10 rows 191
+    // against 209)
+    const int64_t two_from = (L->vdt == MOE_GGML_Q8K ? 13 : 16) * L->E;
     pl.slot_tiles = (T * L->k > 34 * L->E) ? 4 : (T * L->k > two_from) ? 2 : 1;
     if (sw.slot_tiles) pl.slot_tiles = sw.slot_tiles;
     // small batches: slots are numbered t*k + r and no dispatch pass runs; every workgroup then finds its expert's slots
