@@ -13,6 +13,7 @@
 // unsigned as stored.
 #include "act_quant.hpp"
 #include "kernels.hpp"
+#include "lds_dma.hpp"
 #include "slots.hpp"
 
 namespace moe {
@@ -964,13 +965,6 @@ struct alignas(16) QGemmLds {
     alignas(16) float yd[2][QG_NOP * 16][4];          // [buffer][slot][block of the step]
     alignas(16) int bs[2][QG_NOP * 16][4];            // the blocks' sums of quants (formats with a code offset)
 };
-__device__ __forceinline__ uint32_t qg_lds_address(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-// direct global -> LDS load: lane i of the wave writes 16 bytes at lds + 16 i (the issuing wave waits for it with vmcnt)
-__device__ __forceinline__ void qg_dma16(const void* gbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(gbase), "s"(lds));
-}
 
 // WOPS (MODE 1): 16-slot operands per wave.  With 4 the eight waves hold eight weight operands (128 rows) and every one of
 // them takes the tile's four slot operands; with 2 (1) they hold four (two) weight operands, 64 (32) rows, and split
@@ -1028,9 +1022,9 @@ __global__ __launch_bounds__(QG_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
     const uint32_t q_src = (uint32_t)act_row(pos_of_row(16 * (wave >> 1) + (lane & 15))) * (uint32_t)K + (uint32_t)((4 * (wave & 1) + (lane >> 4)) * 16);
     const uint32_t d_src = (uint32_t)act_row(pos_of_row(lane)) * (uint32_t)nkb * 4u;
     auto stage = [&](int ks, int buf) {
-        qg_dma16(ab.qs, q_src + (uint32_t)(ks * 128), qg_lds_address(&L.q[buf][wave >> 1][4 * (wave & 1)][0]));
-        if (wave == 0) qg_dma16(ab.d, d_src + (uint32_t)(ks * 16), qg_lds_address(&L.yd[buf][0][0]));
-        if (WORDS && wave == 1) qg_dma16(ab.bsum, d_src + (uint32_t)(ks * 16), qg_lds_address(&L.bs[buf][0][0]));
+        dma16(ab.qs, q_src + (uint32_t)(ks * 128), lds_address(&L.q[buf][wave >> 1][4 * (wave & 1)][0]));
+        if (wave == 0) dma16(ab.d, d_src + (uint32_t)(ks * 16), lds_address(&L.yd[buf][0][0]));
+        if (WORDS && wave == 1) dma16(ab.bsum, d_src + (uint32_t)(ks * 16), lds_address(&L.bs[buf][0][0]));
     };
 
     const GroupWeights gw = p.groups[grp];

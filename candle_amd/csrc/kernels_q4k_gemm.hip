@@ -50,6 +50,7 @@
 #include <type_traits>
 #include "act_quant.hpp"
 #include "kernels.hpp"
+#include "lds_dma.hpp"
 #include "planes.hpp"
 
 namespace moe {
@@ -91,20 +92,7 @@ struct alignas(16) GemmLds {
     alignas(16) float yd[2][NOP * 16];
 };
 
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-// Direct global->LDS loads: lane i of the wave writes SIZE bytes at lds + SIZE*i; nothing passes through
-// registers, so a whole super-block of activations can be in flight while the wave computes.  The
-// compiler does not see these loads: the issuing wave waits for them (vmcnt) before the barrier that
-// publishes the buffer.
-__device__ __forceinline__ void dma16(const void* gbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(gbase), "s"(lds));
-}
-__device__ __forceinline__ void dma4(const void* gbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(gbase), "s"(lds));
-}
-__device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0)
+__device__ __forceinline__ void wait_all_loads() { wait_loads<0>(); }
 
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(const F& f) {
@@ -198,16 +186,17 @@ __device__ __forceinline__ BPlanes b_prepare(const BRegs& b, int lane) {
     const uint32_t sc47 = (u2 & M4) | (((u0 >> 6) & 0x03030303u) << 4);
     const uint32_t m03 = u1 & 0x3f3f3f3fu;
     const uint32_t m47 = ((u2 >> 4) & M4) | (((u1 >> 6) & 0x03030303u) << 4);
-    // scales split into two 3-bit digits, still one byte per sub-block
-    const uint32_t lo03 = sc03 & 0x07070707u, hi03 = (sc03 >> 3) & 0x07070707u;
-    const uint32_t lo47 = sc47 & 0x07070707u, hi47 = (sc47 >> 3) & 0x07070707u;
+    // scales split into two 3-bit digits, one per 16-bit lane (which the packed multiply takes for both of its halves): scales 0
+    // and 2, 1 and 3, 4 and 6, 5 and 7
+    const uint32_t M7 = 0x00070007u;
+    const uint32_t dl[4] = {sc03 & M7, (sc03 >> 8) & M7, sc47 & M7, (sc47 >> 8) & M7};
+    const uint32_t dh[4] = {(sc03 >> 3) & M7, (sc03 >> 11) & M7, (sc47 >> 3) & M7, (sc47 >> 11) & M7};
 #pragma unroll
     for (int P = 0; P < 4; P++) {
         const u32x4 c = b.c[P >> 1];
         const uint32_t w0 = (P & 1) ? c.z : c.x, w1 = (P & 1) ? c.w : c.y;
-        const uint32_t lw = (P < 2) ? lo03 : lo47, hw = (P < 2) ? hi03 : hi47;
-        const uint32_t slo_a = (lw >> (16 * (P & 1))) & 0xffu, slo_b = (lw >> (16 * (P & 1) + 8)) & 0xffu;
-        const uint32_t shi_a = (hw >> (16 * (P & 1))) & 0xffu, shi_b = (hw >> (16 * (P & 1) + 8)) & 0xffu;
+        const int at = P & 2, up = 16 * (P & 1);
+        const uint32_t slo_a = dl[at] >> up, slo_b = dl[at + 1] >> up, shi_a = dh[at] >> up, shi_b = dh[at + 1] >> up;
         const uint32_t a0 = w0 & M4, a1 = w1 & M4, b0 = (w0 >> 4) & M4, b1 = (w1 >> 4) & M4;
         o.lo[P] = v4i{(int)scale_bytes(a0, slo_a), (int)scale_bytes(a1, slo_a), (int)scale_bytes(b0, slo_b), (int)scale_bytes(b1, slo_b)};
         o.hi[P] = v4i{(int)scale_bytes(a0, shi_a), (int)scale_bytes(a1, shi_a), (int)scale_bytes(b0, shi_b), (int)scale_bytes(b1, shi_b)};
