@@ -29,6 +29,7 @@
 
 #include "act_quant.hpp"
 #include "kernels.hpp"
+#include "lds_dma.hpp"
 #include "planes.hpp"
 #include "slots.hpp"
 
@@ -199,16 +200,18 @@ __device__ inline Q4KPlanes q4k_planes(const Q4KTile& w, int g) {
     const uint32_t sc47 = (u2 & M4) | (((u0 >> 6) & 0x03030303u) << 4);
     const uint32_t m03 = u1 & 0x3f3f3f3fu;
     const uint32_t m47 = ((u2 >> 4) & M4) | (((u1 >> 6) & 0x03030303u) << 4);
+    // the 3-bit digits of the scales, one per 16-bit lane (which the packed multiply takes for both of its halves): scales 0
+    // and 2, 1 and 3, 4 and 6, 5 and 7
+    const uint32_t M7 = 0x00070007u;
+    const uint32_t dl[4] = {sc03 & M7, (sc03 >> 8) & M7, sc47 & M7, (sc47 >> 8) & M7};
+    const uint32_t dh[4] = {(sc03 >> 3) & M7, (sc03 >> 11) & M7, (sc47 >> 3) & M7, (sc47 >> 11) & M7};
     const uint32_t qw[8] = {w.q0.x, w.q0.y, w.q0.z, w.q0.w, w.q1.x, w.q1.y, w.q1.z, w.q1.w};
 #pragma unroll
     for (int P = 0; P < 4; P++) {
         const uint32_t wx = qw[2 * P], wy = qw[2 * P + 1];
         const uint32_t lx = wx & M4, ly = wy & M4, hx = (wx >> 4) & M4, hy = (wy >> 4) & M4;
-        // the digits of four scales at a time, then one bit-field extract per digit
-        const uint32_t scw = (P < 2) ? sc03 : sc47;
-        const uint32_t hiw = (scw >> 3) & 0x07070707u, low = scw & 0x07070707u;
-        const uint32_t s0h = (hiw >> (16 * (P & 1))) & 0xffu, s1h = (hiw >> (16 * (P & 1) + 8)) & 0xffu;
-        const uint32_t s0l = (low >> (16 * (P & 1))) & 0xffu, s1l = (low >> (16 * (P & 1) + 8)) & 0xffu;
+        const int o = P & 2, up = 16 * (P & 1);
+        const uint32_t s0h = dh[o] >> up, s1h = dh[o + 1] >> up, s0l = dl[o] >> up, s1l = dl[o + 1] >> up;
         pl.hi[P] = v4i{(int)digit_times_codes(lx, s0h), (int)digit_times_codes(ly, s0h), (int)digit_times_codes(hx, s1h), (int)digit_times_codes(hy, s1h)};
         pl.lo[P] = v4i{(int)digit_times_codes(lx, s0l), (int)digit_times_codes(ly, s0l), (int)digit_times_codes(hx, s1l), (int)digit_times_codes(hy, s1l)};
     }
@@ -729,6 +732,199 @@ __device__ inline void q4k_up_body(const ExpertParams& p, float (*hbuf)[HBUF_STR
 }
 
 // ---------------------------------------------------------------------------------------------
+// Up projection of Q4K with two slot tiles per pass (lists of 17 to 32 slots).  A workgroup owns 256 rows of F of one expert as
+// above, with eight waves of two row tiles of w1 and two of w3.  Their 32 activation rows are the same: a super-block of them
+// goes into LDS once (double-buffered, direct loads, one barrier per super-block) instead of into every wave's registers, and a
+// weight tile is unpacked pair by pair between the matrix instructions, so that a wave needs 126 registers and four of them
+// share a SIMD.
+// What bounds it: vector instructions, 154 per tile and two operands (90 unpack it, 64 add up results with the reference's roundings)
+// beside 18 matrix instructions, and 448 workgroups on 256 CUs.  Up launch, Mixtral shape, four waves of eight tiles at two per SIMD with
+// the rows in registers / this: 56 tokens 117 / 110 us, 100 tokens 126 / 118, 136 tokens 176 / 163; a quarter of its width, 100 tokens
+// 26.1 / 22.4.  (Q5K unpacks faster sub-block by sub-block than into planes, 108 / 142 here; Q6K measured the same both ways.)
+struct Up2Q4K {
+    typedef Q4KTile Tile;
+    static constexpr int TILE_BYTES = Q4K_TILE_BYTES, LOADS = 3;
+    static constexpr bool kSums = true;
+    struct Scales {
+        float d, dmin;
+        // the 3-bit digits of the eight scales, one per 16-bit lane (a lane is what the packed multiply can take twice):
+        // [0], [1]: scales 0 and 2, 1 and 3; [2], [3]: 4 and 6, 5 and 7
+        uint32_t hi[4], lo[4];
+        v4h mB;
+    };
+    static __device__ __forceinline__ Tile load(const uint8_t* tile, int lane) { return load_q4k_tile(tile, lane); }
+    // low_half: all ones in lane groups 0 and 1, whose block sums belong to the first four sub-blocks (a mask: a branch would end
+    // the loop's basic block)
+    static __device__ __forceinline__ Scales scales(const Tile& w, int g, uint32_t low_half) {
+        const uint32_t M4 = 0x0f0f0f0fu, M7 = 0x00070007u;
+        const uint32_t u0 = w.sc.y, u1 = w.sc.z, u2 = w.sc.w;
+        Scales S;
+        S.d = __half2float(__ushort_as_half((unsigned short)(w.sc.x & 0xffffu)));
+        S.dmin = __half2float(__ushort_as_half((unsigned short)(w.sc.x >> 16)));
+        const uint32_t sc03 = u0 & 0x3f3f3f3fu, sc47 = (u2 & M4) | (((u0 >> 6) & 0x03030303u) << 4);
+        S.lo[0] = sc03 & M7; S.lo[1] = (sc03 >> 8) & M7; S.lo[2] = sc47 & M7; S.lo[3] = (sc47 >> 8) & M7;
+        S.hi[0] = (sc03 >> 3) & M7; S.hi[1] = (sc03 >> 11) & M7; S.hi[2] = (sc47 >> 3) & M7; S.hi[3] = (sc47 >> 11) & M7;
+        const uint32_t m03 = u1 & 0x3f3f3f3fu, m47 = ((u2 >> 4) & M4) | (((u1 >> 6) & 0x03030303u) << 4);
+        const uint32_t mw = (m03 & low_half) | (m47 & ~low_half);
+        const _Float16 ma = (_Float16)(int)((mw >> (16 * (g & 1))) & 0xffu), mb = (_Float16)(int)((mw >> (16 * (g & 1) + 8)) & 0xffu);
+        S.mB = v4h{ma, ma, mb, mb};
+        return S;
+    }
+    template <int P>
+    static __device__ __forceinline__ void planes(const Tile& w, const Scales& S, int, v4i& hi, v4i& lo) {
+        const uint32_t M4 = 0x0f0f0f0fu;
+        const uint4& q = P < 2 ? w.q0 : w.q1;
+        const uint32_t wx = P & 1 ? q.z : q.x, wy = P & 1 ? q.w : q.y;
+        const uint32_t lx = wx & M4, ly = wy & M4, hx = (wx >> 4) & M4, hy = (wy >> 4) & M4;
+        const int o = P & 2, up = 16 * (P & 1);
+        const uint32_t s0h = S.hi[o] >> up, s1h = S.hi[o + 1] >> up, s0l = S.lo[o] >> up, s1l = S.lo[o + 1] >> up;
+        hi = v4i{(int)digit_times_codes(lx, s0h), (int)digit_times_codes(ly, s0h), (int)digit_times_codes(hx, s1h), (int)digit_times_codes(hy, s1h)};
+        lo = v4i{(int)digit_times_codes(lx, s0l), (int)digit_times_codes(ly, s0l), (int)digit_times_codes(hx, s1l), (int)digit_times_codes(hy, s1l)};
+    }
+    // (rounded where q4k_mac_planes rounds)
+    static __device__ __forceinline__ void result(const Scales& S, int hi, int lo, float Dm, float yd, float& acc) {
+        acc += (S.d * yd) * (float)(8 * hi + lo);
+        acc -= (S.dmin * yd) * Dm;
+    }
+};
+struct Up2Stage {
+    uint8_t q[2][2][4][1024];            // [buffer][slot tile][pair][lane] 16 bytes: an operand of one matrix instruction
+    _Float16 bs[2][2][2][16][8];         // [buffer][slot tile][half][slot] eight block sums
+    float yd[2][64];                     // [buffer][slot] (two copies of the 32)
+};
+template <class FMT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void q4k_up2_kernel(ExpertParams p) {
+    constexpr int NW = 8, RTW = 2, NT = 2 * RTW, RING = 1;
+    __shared__ __align__(16) uint8_t lds[sizeof(Up2Stage) > 32 * HBUF_STRIDE * 4 ? sizeof(Up2Stage) : 32 * HBUF_STRIDE * 4];
+    __shared__ int list_lds[DIRECT_MAX_SLOTS];
+    __shared__ int wtot_lds[NW];
+    Up2Stage& L = *reinterpret_cast<Up2Stage*>(lds);
+    float (*hbuf)[HBUF_STRIDE] = reinterpret_cast<float (*)[HBUF_STRIDE]>(lds);   // the K loop is done with the staging buffers then
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = blockIdx.y;
+    const int H = p.H, F = p.F, nsb = H / 256, rb = blockIdx.x;
+    const GroupWeights gw = p.groups[grp];
+    const int rt0 = rb * 16 + wave * RTW;
+    const uint8_t* tp[NT];
+#pragma unroll
+    for (int j = 0; j < RTW; j++) {
+        tp[j] = gw.w1 + (size_t)(rt0 + j) * FMT::TILE_BYTES;
+        tp[RTW + j] = gw.w3 + (size_t)(rt0 + j) * FMT::TILE_BYTES;
+    }
+    const size_t sb_stride = (size_t)(F / 16) * FMT::TILE_BYTES;
+    if (blockIdx.z > 0 && !p.rb.direct && !p.is_shared) {   // (a later pass: see q4k_up_body)
+        const int gi = p.group0 + grp;
+        if ((int)blockIdx.z * 32 >= p.rb.offsets[gi + 1] - p.rb.offsets[gi]) return;
+    }
+    // first weight tiles go out before anything else; an expert without tokens wastes them
+    typename FMT::Tile ring[RING];
+#pragma unroll
+    for (int j = 0; j < RING; j++) ring[j] = FMT::load(tp[j], lane);
+    const GroupSlots gs = group_slots<NW * 64>(p, grp, list_lds, wtot_lds);
+    const int tg0 = blockIdx.z * 32;
+    if (tg0 >= gs.n) return;
+    auto act_row = [&](int i) { return (uint32_t)slot_token(p, gs.slot(tg0 + i < gs.n ? tg0 + i : gs.n - 1)); };
+    // wave w stages pair w % 4 of slot tile w / 4, wave 0 also the block sums and wave 1 the scales
+    const uint32_t q_src = act_row((wave >> 2) * 16 + r) * (uint32_t)H + (uint32_t)((wave & 3) * 64 + g * 16);
+    const uint32_t s_src = wave == 0 ? (act_row((lane >> 5) * 16 + r) * (uint32_t)nsb * 16 + (uint32_t)(g & 1) * 8) * 2 : act_row(lane & 31) * (uint32_t)nsb * 4;
+    auto stage = [&](int sb, int buf) {
+        dma16(p.xq.qs + sb * 256, q_src, lds_address(&L.q[buf][wave >> 2][wave & 3][0]));
+        if (FMT::kSums && wave == 0) dma16(static_cast<const uint8_t*>(p.xq.bsum) + sb * 32, s_src, lds_address(&L.bs[buf][0][0][0][0]));
+        if (wave == 1) dma4(p.xq.d + sb, s_src, lds_address(&L.yd[buf][0]));
+    };
+    stage(0, 0);
+    wait_loads<0>();
+    __syncthreads();
+
+    uint32_t low_half = g < 2 ? ~0u : 0u;
+    asm volatile("" : "+v"(low_half));
+    // a pass over a list that ends inside its first slot tile multiplies that one only (wave-uniform)
+    auto run = [&](auto ttl_tag) {
+        constexpr int TTL = decltype(ttl_tag)::value;
+        float acc[NT][TTL][4];
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int tt = 0; tt < TTL; tt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[j][tt][i] = 0.f;
+        for (int sb = 0; sb < nsb; sb++) {
+            const int buf = sb & 1;
+            if (sb + 1 < nsb) stage(sb + 1, buf ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const typename FMT::Tile w = ring[j % RING];
+                const int jn = (j + RING) % NT;
+                int sbn = sb + (j + RING) / NT;
+                sbn = sbn < nsb ? sbn : nsb - 1;
+                ring[j % RING] = FMT::load(tp[jn] + (size_t)sbn * sb_stride, lane);
+                __builtin_amdgcn_sched_barrier(0);
+                const typename FMT::Scales S = FMT::scales(w, g, low_half);
+                const v4i zero = {0, 0, 0, 0};
+                v4i hi[TTL], lo[TTL];
+                auto pair = [&](auto p_tag) {
+                    constexpr int P = decltype(p_tag)::value;
+                    v4i wh, wl;
+                    FMT::template planes<P>(w, S, g, wh, wl);
+#pragma unroll
+                    for (int tt = 0; tt < TTL; tt++) {
+                        const v4i a = *reinterpret_cast<const v4i*>(&L.q[buf][tt][P][lane * 16]);
+                        hi[tt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, wh, P == 0 ? zero : hi[tt], 0, 0, 0);
+                        lo[tt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, wl, P == 0 ? zero : lo[tt], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);   // (a pair at a time, for the sake of the registers)
+                };
+                pair(std::integral_constant<int, 0>{}); pair(std::integral_constant<int, 1>{});
+                pair(std::integral_constant<int, 2>{}); pair(std::integral_constant<int, 3>{});
+#pragma unroll
+                for (int tt = 0; tt < TTL; tt++) {
+                    v4f Dm = {0.f, 0.f, 0.f, 0.f};
+                    if constexpr (FMT::kSums)
+                        Dm = __builtin_amdgcn_mfma_f32_16x16x16f16(*reinterpret_cast<const v4h*>(&L.bs[buf][tt][g >> 1][r][(g & 1) * 4]), S.mB, Dm, 0, 0, 0);
+                    const v4f yd = *reinterpret_cast<const v4f*>(&L.yd[buf][tt * 16 + 4 * g]);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) FMT::result(S, hi[tt][i], lo[tt][i], Dm[i], yd[i], acc[j][tt][i]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            wait_loads<RING * FMT::LOADS>();   // all but the two weight tiles requested last: the staged rows have landed
+            __syncthreads();
+        }
+        // h = silu(w1 x) * (w3 x), then the 256-row block of every slot is quantised (as in q4k_up_body)
+#pragma unroll
+        for (int tt = 0; tt < TTL; tt++)
+#pragma unroll
+            for (int j = 0; j < RTW; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    hbuf[tt * 16 + 4 * g + i][(wave * RTW + j) * 16 + r] = silu_fast(acc[j][tt][i]) * acc[RTW + j][tt][i];
+        __syncthreads();
+        const int nfb = F / 256;
+        constexpr int NQ = TTL * 16 / NW;
+        float4 v[NQ];
+        bool valid[NQ];
+        int8_t* qs_out[NQ];
+        float* d_out[NQ];
+        __half* bs_out[NQ];
+#pragma unroll
+        for (int n = 0; n < NQ; n++) {
+            const int tok = wave + n * NW;
+            valid[n] = tg0 + tok < gs.n;
+            v[n] = *reinterpret_cast<const float4*>(&hbuf[tok][lane * 4]);
+            const int64_t hrow = gs.slot(valid[n] ? tg0 + tok : gs.n - 1) - p.slot_origin;
+            qs_out[n] = p.hq.qs + hrow * F + rb * 256;
+            d_out[n] = p.hq.d + hrow * nfb + rb;
+            bs_out[n] = reinterpret_cast<__half*>(p.hq.bsum) + (hrow * nfb + rb) * 16;
+        }
+        quantize_q8k_blocks<NQ>(v, valid, lane, qs_out, d_out, bs_out);
+    };
+    if (gs.n - tg0 <= 16) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
+}
+
+// ---------------------------------------------------------------------------------------------
 // Down projection: a workgroup owns NTD row tiles (64 weight rows; 32 for very small batches) of one
 // expert; its NW waves split K, every wave carrying the tiles over its K range, and the partial sums
 // meet in LDS.
@@ -864,7 +1060,6 @@ __device__ inline void q4k_down_body(const ExpertParams& p, float (*part)[NTD * 
 DEF_UP(q4k_up_t1_v0, FmtQ4K, 1, 8, 2, 4)
 DEF_UP(q4k_up_t1_v1, FmtQ4K, 1, 4, 2, 3)
 DEF_UP_NARROW(q4k_up_t1_narrow, FmtQ4K, 4, 2, 4)   // 127 registers: a fourth wave per SIMD is free (batch 2: 85 -> 80 us per step)
-DEF_UP(q4k_up_t2, FmtQ4KP, 2, 4, 2, 2)
 DEF_UP(q4k_up_t4, FmtQ4KP, 4, 8, 2, 2)
 DEF_DOWN(q4k_down_t1_v0, FmtQ4K, 1, 8, 2, 4)
 DEF_DOWN(q4k_down_t1_v1, FmtQ4K, 1, 4, 2, 3)
@@ -1141,7 +1336,7 @@ struct KernelFamily {
 };
 static const KernelFamily* kernel_family(int dt) {
     static const int uv = variant("MOE_UP_VARIANT", 1), dv = variant("MOE_DOWN_VARIANT", 1);
-    static const KernelFamily q4k = {uv == 0 ? q4k_up_t1_v0 : q4k_up_t1_v1, q4k_up_t1_narrow, q4k_up_t2, q4k_up_t4,
+    static const KernelFamily q4k = {uv == 0 ? q4k_up_t1_v0 : q4k_up_t1_v1, q4k_up_t1_narrow, q4k_up2_kernel<Up2Q4K>, q4k_up_t4,
                                      dv == 0 ? q4k_down_t1_v0 : q4k_down_t1_v1, q4k_down_t1_narrow, q4k_down_t2, q4k_down_t4,
                                      q4k_down_t1_fine, q4k_down_t2_fine, q4k_down_t4_fine};
     static const KernelFamily q2k = {q2k_up_t1, q2k_up_t1_narrow, q2k_up_t2, nullptr, q2k_down_t1, q2k_down_t1_narrow, q2k_down_t2, nullptr,
@@ -1175,7 +1370,7 @@ hipError_t launch_q4k_up(const ExpertParams& p, hipStream_t s) {
     }
     dim3 grid((unsigned)(p.F / 256), (unsigned)p.n_groups, (unsigned)((p.max_rows + tt * 16 - 1) / (tt * 16)));
     if (tt == 4) hipLaunchKernelGGL(f->up_t4, grid, dim3(512), 0, s, p);
-    else if (tt == 2) hipLaunchKernelGGL(f->up_t2, grid, dim3(256), 0, s, p);
+    else if (tt == 2) hipLaunchKernelGGL(f->up_t2, grid, dim3(p.dt == MOE_GGML_Q4K ? 512 : 256), 0, s, p);
     else hipLaunchKernelGGL(f->up_t1, grid, dim3(p.dt == MOE_GGML_Q4K && uv == 0 ? 512 : 256), 0, s, p);
     return hipGetLastError();
 }
