@@ -1118,53 +1118,52 @@ __global__ __launch_bounds__(QG_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4
     const int n = lane & 15;
     if (MODE == 0) {
         // Wave w < 4 holds w1 x of 16 rows, wave w + 4 holds w3 x of the same rows.  Each of the two parks half of its sums
-        // in LDS (the staging buffers are free now) and combines the other half: the w1 wave slot operands 0 and 1, the
-        // w3 wave operands 2 and 3 -- a wave's silu evaluations are a chain of dependent double-precision operations, and
-        // eight waves carry eight of them each instead of four waves sixteen.
-        float* xch = reinterpret_cast<float*>(&L.q[0][0][0][0]);   // [8 waves][2 operands][4 i][64 lanes] floats
-        static_assert(8 * 2 * 4 * 64 * 4 <= sizeof(L.q) && QG_NOP == 4, "exchange area");
+        // in LDS (the staging buffers are free now) and combines the other half: the w1 wave result registers 0 and 2, the
+        // w3 wave registers 1 and 3 -- a wave's silu evaluations are a chain of dependent double-precision operations, and
+        // eight waves carry eight of them each instead of four waves sixteen.  Registers beyond the end of the list are left
+        // out, and so are its slots below: both halves follow the list length, evenly over the waves.  (Qwen-MoE shape, Q8_0, us per
+        // layer, 64 slots' epilogue for every tile / this: 310 tokens 240 / 223, 512 tokens 275 / 270, 1000 tokens 427 / 411, 2000
+        // tokens 741 / 719.)
+        float* xch = reinterpret_cast<float*>(&L.q[0][0][0][0]);   // [8 waves][4 operands][2 registers][64 lanes] floats
+        static_assert(8 * 4 * 2 * 64 * 4 <= sizeof(L.q) && QG_NOP == 4, "exchange area");
+        const int odd = wave >> 2;
 #pragma unroll
-        for (int oo = 0; oo < 2; oo++)
+        for (int o = 0; o < QG_NOP; o++)
+            if (o < n_op) {   // wave-uniform
 #pragma unroll
-            for (int i = 0; i < 4; i++) xch[((wave * 2 + oo) * 4 + i) * 64 + lane] = wave < 4 ? acc[2 + oo][i] : acc[oo][i];
+                for (int h = 0; h < 2; h++) xch[((wave * QG_NOP + o) * 2 + h) * 64 + lane] = odd ? acc[o][2 * h] : acc[o][2 * h + 1];
+            }
         __syncthreads();
         const int partner = wave ^ 4;
 #pragma unroll
-        for (int oo = 0; oo < 2; oo++)
+        for (int o = 0; o < QG_NOP; o++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float other = xch[((partner * 2 + oo) * 4 + i) * 64 + lane];
-                const int o = (wave < 4 ? 0 : 2) + oo;
-                // silu(w1 x) * (w3 x): the operand this wave kept, times / under the partner's
-                const float gate_v = wave < 4 ? acc[oo][i] : other, up_v = wave < 4 ? other : acc[2 + oo][i];
-                hx[o * 16 + 4 * i + g][(wave & 3) * 16 + n] = silu_ref32(gate_v, exp_tab) * up_v;
+            for (int h = 0; h < 2; h++) {
+                const int pos = o * 16 + 4 * (2 * h + odd);   // of lane group 0
+                if (pos < n_here) {   // wave-uniform
+                    const float other = xch[((partner * QG_NOP + o) * 2 + h) * 64 + lane];
+                    const float mine = odd ? acc[o][2 * h + 1] : acc[o][2 * h];
+                    // silu(w1 x) * (w3 x): the register this wave kept, times / under the partner's
+                    hx[pos + g][(wave & 3) * 16 + n] = silu_ref32(odd ? other : mine, exp_tab) * (odd ? mine : other);
+                }
             }
         __syncthreads();
         // Q8_0 blocks of h (BlockQ8_0::from_float, k_quants.rs:605-634): the workgroup's 64 rows are two blocks per slot;
         // half a wave quantises one (slot, block)
-        const int nfb = p.F / 32;
-#pragma unroll
-        for (int it = 0; it < QG_NOP * 16 * 2 / 16; it++) {
-            const int pair = (wave * (QG_NOP * 2) + it) * 2 + (lane >> 5);
-            const int slot_in_tile = pair >> 1, blk = pair & 1, e = lane & 31;
-            const float x = hx[slot_in_tile][blk * 32 + e];
-            float amax = fabsf(x);
-#pragma unroll
-            for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+        const int nfb = p.F / 32, blk = lane >> 5, e = lane & 31;
+        for (int slot_in_tile = wave; slot_in_tile < n_here; slot_in_tile += 8) {
+            const float x = hx[slot_in_tile][lane];
+            const float amax = block32_max(fabsf(x));
             const float d = amax / 127.0f;
             const float id = (d != 0.f) ? 1.0f / d : 0.f;
             const int q = round_as_i8(x * id);
-            int sum = q;
-#pragma unroll
-            for (int o = 16; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-            if (slot_in_tile < n_here) {
-                const int64_t hrow = s_begin + pos0 + slot_in_tile - p.slot_origin;
-                p.hq.qs[hrow * p.F + rblk * 64 + blk * 32 + e] = (int8_t)q;
-                if (e == 0) {
-                    const float dh = __half2float(__float2half_rn(d));
-                    p.hq.d[hrow * nfb + rblk * 2 + blk] = dh;
-                    reinterpret_cast<int32_t*>(p.hq.bsum)[hrow * nfb + rblk * 2 + blk] = q8_block_word(vecdot_dtype(DT), sum, dh);
-                }
+            const int sum = block32_sum(q);
+            const int64_t hrow = s_begin + pos0 + slot_in_tile - p.slot_origin;
+            p.hq.qs[hrow * p.F + rblk * 64 + lane] = (int8_t)q;
+            if (e == 0) {
+                const float dh = __half2float(__float2half_rn(d));
+                p.hq.d[hrow * nfb + rblk * 2 + blk] = dh;
+                reinterpret_cast<int32_t*>(p.hq.bsum)[hrow * nfb + rblk * 2 + blk] = q8_block_word(vecdot_dtype(DT), sum, dh);
             }
         }
     } else {

@@ -889,7 +889,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            wait_loads<RING * FMT::LOADS>();   // all but the two weight tiles requested last: the staged rows have landed
+            wait_loads<RING * FMT::LOADS>();   // all but the weight tile requested last: the staged rows have landed
             __syncthreads();
         }
         // h = silu(w1 x) * (w3 x), then the 256-row block of every slot is quantised (as in q4k_up_body)
