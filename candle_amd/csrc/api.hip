@@ -537,7 +537,10 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
     }
     // Q8_0 / Q4_0 / Q5_0 layers whose slots are grouped by expert (more than DIRECT_MAX_SLOTS assignments): the tiled
     // kernels of kernels_q32.hip read an expert's weights once for up to 64 of its slots
-    pl.tiled32 = !sw.no_gemm && !pl.direct && q8_0_gemm_usable(L->dt, L->dt_down, L->H, L->F) && T * L->k > 20 * L->E;
+    // (Many experts: from 11 rows per expert on -- the lists are short of a tile, but a streaming launch over a measured list holds a
+    // workgroup for every pass a list could need, most of them empty.  Qwen-MoE shape, Q8_0, streamed / tiled: 120 tokens, 8 rows
+    // per expert, 191 / 218 us, 150 tokens 195 / 195, 180 tokens 216 / 205, 210 tokens 240 / 200, 240 tokens 258 / 210)
+    pl.tiled32 = !sw.no_gemm && !pl.direct && q8_0_gemm_usable(L->dt, L->dt_down, L->H, L->F) && T * L->k > (L->E > 16 ? 11 : 20) * L->E;
     if (pl.tiled32) pl.tile_slots = 64;
     return pl;
 }
