@@ -537,10 +537,12 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
     }
     // Q8_0 / Q4_0 / Q5_0 layers whose slots are grouped by expert (more than DIRECT_MAX_SLOTS assignments): the tiled
     // kernels of kernels_q32.hip read an expert's weights once for up to 64 of its slots
-    // (Many experts: from 11 rows per expert on -- the lists are short of a tile, but a streaming launch over a measured list holds a
-    // workgroup for every pass a list could need, most of them empty.  Qwen-MoE shape, Q8_0, streamed / tiled: 120 tokens, 8 rows
-    // per expert, 191 / 218 us, 150 tokens 195 / 195, 180 tokens 216 / 205, 210 tokens 240 / 200, 240 tokens 258 / 210)
-    pl.tiled32 = !sw.no_gemm && !pl.direct && q8_0_gemm_usable(L->dt, L->dt_down, L->H, L->F) && T * L->k > (L->E > 16 ? 11 : 20) * L->E;
+    // (Many experts: from 13 rows per expert on -- the lists are short of a tile, but a streaming launch over a measured list holds a
+    // workgroup for every pass a list could need, most of them empty.  Streamed / tiled, us, Q8_0: Qwen-MoE shape 120 tokens, 8 rows per
+    // expert, 191 / 218, 170 tokens 204 / 202, 220 tokens 250 / 200, 300 tokens 243 / 220; without its always-on expert 170 tokens
+    // 145 / 159, 220 tokens 175 / 155; 32 experts of 4096 x 4096, top-2, 240 tokens, 15 rows, 433 / 345, 300 tokens 373 / 379; 128 experts
+    // of 1024 x 512, top-8, 180 tokens, 11 rows, 92 / 82.  Up to 16 experts: Mixtral shape, Q4_0, 60 tokens, 15 rows, 219 / 247.)
+    pl.tiled32 = !sw.no_gemm && !pl.direct && q8_0_gemm_usable(L->dt, L->dt_down, L->H, L->F) && T * L->k > (L->E > 16 ? 13 : 20) * L->E;
     if (pl.tiled32) pl.tile_slots = 64;
     return pl;
 }
