@@ -404,8 +404,7 @@ struct Q32SStage {
     float d[TT];
     int w[TT];
 };
-// Requests step ks of the activations.  A step past the end of K (the K loop runs in whole rounds of its prefetch
-// ring) re-reads the last one; q32s_commit zeroes its scale and word, so that its products add +-0.  (Nothing here
+// Requests step ks of the activations; past the end of K the last one is requested again and never used.  (Nothing here
 // may touch the loaded values: that would wait for the loads where they are issued.)
 template <int TT>
 __device__ __forceinline__ void q32s_issue(Q32SStage<TT>& st, const Q32SRows<TT>& rows, const ActBuf& ab, int K, int nkb, int ks, int tid) {
@@ -427,7 +426,7 @@ __device__ __forceinline__ void q32s_issue(Q32SStage<TT>& st, const Q32SRows<TT>
 constexpr int Q32S_MAGIC_BITS = 0x4B400000;
 constexpr float Q32S_MAGIC = 12582912.0f;
 template <int TT, int OFFSET>
-__device__ __forceinline__ void q32s_commit(const Q32SStage<TT>& st, uint8_t* buf, int tid, bool past) {
+__device__ __forceinline__ void q32s_commit(const Q32SStage<TT>& st, uint8_t* buf, int tid) {
     const int slot = tid >> 4, c = tid & 15, b = c >> 2, cc = c & 3;
     // elements 8cc .. 8cc+3 of the block belong to chunk g0 = 2 (cc % 2), the next four to chunk g0 + 1; both are the
     // low (cc < 2) or the high half of their lane's operand
@@ -438,8 +437,8 @@ __device__ __forceinline__ void q32s_commit(const Q32SStage<TT>& st, uint8_t* bu
         *reinterpret_cast<uint32_t*>(base + at) = st.q[tt].x;
         *reinterpret_cast<uint32_t*>(base + at + 128) = st.q[tt].y;
         const int at_s = Q32S_ACT_Q + ((tid & 3) * 16 + ((tid >> 2) & 15)) * 4;   // [block][slot] scales, then words
-        *reinterpret_cast<float*>(base + at_s) = past ? 0.f : st.d[tt];
-        *reinterpret_cast<int*>(base + at_s + 256) = OFFSET ? Q32S_MAGIC_BITS - st.w[tt] * OFFSET : (past ? 0 : st.w[tt]);
+        *reinterpret_cast<float*>(base + at_s) = st.d[tt];
+        *reinterpret_cast<int*>(base + at_s + 256) = OFFSET ? Q32S_MAGIC_BITS - st.w[tt] * OFFSET : st.w[tt];
     }
 }
 
@@ -497,13 +496,19 @@ __device__ __forceinline__ void q32s_engine(const uint8_t* const tp[NT], size_t 
 #pragma unroll
         for (int t = 0; t < NT; t++) ring[j][t] = load_q32s<DT, ONCE>(tp[t] + (size_t)(j < nks ? j : nks - 1) * stride, lane);
     }
-    q32s_commit<TT, Q32Fmt<DT>::OFFSET>(st[0], act_lds, tid, false);
+    q32s_commit<TT, Q32Fmt<DT>::OFFSET>(st[0], act_lds, tid);
     q32s_issue<TT>(st[0], rows, ab, K, nkb, D, tid);
     __syncthreads();
-    for (int ks0 = 0; ks0 < nks; ks0 += D) {
+    // A last round that is not full ends early: its surplus steps would multiply the last tile again, and even by zero scales an
+    // infinite minimum is no number then.  (Two steps deep the odd one follows the loop instead: a branch in it costs the two-tile
+    // kernels up to 2 %, six deep the steps behind it cost registers.  Q8_0, us before / after: 25664 x 3200, 25 steps, 12 rows 25.2 / 22.5;
+    // 8192 x 1408, 11 steps, 64 rows 14.7 / 13.7; 4096 x 4096, 32 steps, 200 rows 36.2 / 36.3.)
+    const int nks_loop = D == 2 ? nks & ~1 : nks;
+    for (int ks0 = 0; ks0 < nks_loop; ks0 += D) {
 #pragma unroll
         for (int j = 0; j < D; j++) {
             const int ks = ks0 + j;
+            if (D > 2 && j > 0 && ks >= nks) break;   // uniform
             Q32SRaw<DT> cur[NT];
             const int ksn = ks + D < nks ? ks + D : nks - 1;
 #pragma unroll
@@ -517,10 +522,18 @@ __device__ __forceinline__ void q32s_engine(const uint8_t* const tp[NT], size_t 
             __builtin_amdgcn_sched_barrier(0);
             // step ks + 1 goes into the other buffer (nobody reads it before the barrier below), its ring position
             // takes the request for step ks + 1 + D
-            q32s_commit<TT, Q32Fmt<DT>::OFFSET>(st[(j + 1) % D], act_lds + ((ks + 1) & 1) * (TT * Q32S_ACT_BYTES), tid, ks + 1 >= nks);
+            q32s_commit<TT, Q32Fmt<DT>::OFFSET>(st[(j + 1) % D], act_lds + ((ks + 1) & 1) * (TT * Q32S_ACT_BYTES), tid);
             q32s_issue<TT>(st[(j + 1) % D], rows, ab, K, nkb, ks + 1 + D, tid);
             __syncthreads();
         }
+    }
+    if (D == 2 && nks_loop < nks) {   // uniform
+        const uint8_t* buf = act_lds + (nks_loop & 1) * (TT * Q32S_ACT_BYTES);
+        q32s_step<DT, TT, NT, 0>(ring[0], buf, lane, acc);
+        q32s_step<DT, TT, NT, 1>(ring[0], buf, lane, acc);
+        q32s_step<DT, TT, NT, 2>(ring[0], buf, lane, acc);
+        q32s_step<DT, TT, NT, 3>(ring[0], buf, lane, acc);
+        __syncthreads();
     }
 }
 
