@@ -14,6 +14,7 @@
 #include "act_quant.hpp"
 #include "kernels.hpp"
 #include "lds_dma.hpp"
+#include "q32_plan.hpp"
 #include "slots.hpp"
 
 namespace moe {
@@ -858,27 +859,9 @@ __global__ __launch_bounds__(Q32_THREADS) __attribute__((amdgpu_waves_per_eu(4, 
     }
 }
 
-// When the fine kernels are the faster ones.  Counted in workgroups of the coarse kernels (128 rows of F, 64 of H) over passes of 16
-// slots that find slots: up to 700 for the up projection, a list's second and later passes counted twice (they read its
-// weights again); up to 400 for the down projection.  Up, us, coarse / fine: a quarter of Mixtral's width, Q4_0, 224 (up to 40 tokens)
-// 16.8 / 14.6, 448 (100 tokens, two passes) 31.4 / 28.0, three passes 32.8 / 37.2; Qwen-MoE shape, Q8_0, 44 (one token) 31 / 15, 176
-// 47 / 21, 660 (16 tokens) 54 / 43, (64 tokens) 67 / 63; Mixtral, Q4_0, 448 (two tokens) 85 / 56, 896 93 / 97.  Down: a quarter of Mixtral's width
-// 32 17.8 / 10.0, 128 19.8 / 12.3, 256 27.3 / 22.7; Mixtral 128 55 / 32, 256 63 / 51, 512 64 / 81; Qwen-MoE shape 256 14.3 / 12.0, 512 18.6 / 18.8;
-// dense Q8_0 4096 x 4096 64 (16 rows) 21.4 / 11.4, 256 27.8 / 18.6, 448 28.4 / 27.7, 512 28.9 / 30.8; 4096 x 14336 320 84 / 77, 448 87 / 95.
-// A one-tile launch some of whose lists may need a second pass stays coarse in the up projection (Q4_0, 64 tokens 20.8 / 22.6).
-struct Q32Passes {
-    int64_t all, first;   // passes that find slots, and those among them that are their list's first
-};
-static Q32Passes q32_passes(const ExpertParams& p) {
-    if (p.n_groups == 1) return Q32Passes{(p.max_rows + 15) / 16, 1};
-    const int64_t slots = (int64_t)p.rb.T * p.rb.k, first = std::min<int64_t>(p.n_groups, slots);
-    return Q32Passes{std::max(gemm_tiles(slots, p.n_groups, 16), first), first};   // (lists as evenly filled as gemm_tiles takes them)
+static Q32Grid q32_grid(const ExpertParams& p) {
+    return p.is_shared ? q32_grid(p.max_rows, 1, 1, false, true) : q32_grid(p.rb.T, p.rb.k, p.n_groups, p.rb.direct != 0, false);
 }
-static bool q32_up_fine(const ExpertParams& p, int slot_tiles) {
-    const Q32Passes n = q32_passes(p);
-    return (p.F / 32 + 3) / 4 * (2 * n.all - n.first) <= 700 && (slot_tiles > 1 || n.all == n.first);
-}
-static bool q32_down_fine(const ExpertParams& p) { return (p.H / 16 + 3) / 4 * q32_passes(p).all <= 400; }
 // The grid of a fine launch: a row of workgroups per assignment where there are fewer of them than experts.
 static dim3 q32_fine_grid(ExpertParams& p, int64_t row_blocks) {
     const int64_t slots = (int64_t)p.rb.T * p.rb.k;
@@ -902,7 +885,7 @@ static hipError_t launch_q32_up_t(const ExpertParams& p, hipStream_t s) {
     const int wpb = Q32_THREADS / 64;
     const int n_pairs = p.F / 32;
     dim3 grid((unsigned)((n_pairs + wpb - 1) / wpb), (unsigned)p.n_groups, (unsigned)((p.max_rows + tt * 16 - 1) / (tt * 16)));
-    if (stream && q32_up_fine(p, tt)) {
+    if (stream && q32_up_fine(p.F, q32_grid(p), tt)) {
         ExpertParams q = p;
         const dim3 fine = q32_fine_grid(q, n_pairs);
         hipLaunchKernelGGL((q32s_up_fine_kernel<DT, 2>), fine, dim3(Q32_THREADS), 0, s, q);
@@ -937,7 +920,7 @@ static hipError_t launch_q32_down_t(const ExpertParams& p, hipStream_t s) {
     const int tt = p.slot_tiles >= 2 ? 2 : 1;
     const int wpb = Q32_THREADS / 64;
     dim3 grid((unsigned)((p.H / 16 + wpb - 1) / wpb), (unsigned)p.n_groups, (unsigned)((p.max_rows + tt * 16 - 1) / (tt * 16)));
-    if (stream && q32_down_fine(p)) {
+    if (stream && q32_down_fine(p.H, q32_grid(p))) {
         ExpertParams q = p;
         const dim3 fine = q32_fine_grid(q, p.H / 16);
         hipLaunchKernelGGL((q32s_down_fine_kernel<DT, 2>), fine, dim3(Q32_THREADS), 0, s, q);

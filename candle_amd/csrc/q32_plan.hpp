@@ -1,0 +1,53 @@
+// Which kernels a streaming launch of the 32-element formats takes: workgroups of a quarter of the rows ("fine") or whole ones.
+// Plain C++: no HIP types.
+//
+// The lines are those of 10962 measured (layer, tokens) pairs: 1160 random layers of 4 to 256 experts (H 256 .. 4096, F 128 .. 8192, top-1
+// to top-10, the five formats, with and without an always-on expert), 0.05 to 33 rows per expert, every variant timed at each.
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+#include "gemm_plan.hpp"
+
+namespace moe {
+
+// What a streaming launch's grid holds, in passes of 16 slots.
+struct Q32Grid {
+    enum Kind { ROWS, DIRECT, LISTS, ALWAYS_ON } kind;   // one list alone; lists found by scanning the assignments; lists measured by a dispatch pass; the always-on expert, beside the routed launches
+    int64_t live, first;   // passes that find slots, and those among them that are their list's first
+    int64_t empty;         // passes that find none, in the grid of a fine launch: the host knows no list's length
+};
+// groups: lists (one for a dense product); direct: no dispatch pass ran
+inline Q32Grid q32_grid(int64_t T, int64_t k, int64_t groups, bool direct, bool always_on) {
+    const int64_t z = (T + 15) / 16;
+    if (always_on || groups == 1) return Q32Grid{always_on ? Q32Grid::ALWAYS_ON : Q32Grid::ROWS, z, 1, 0};
+    const int64_t slots = T * k, first = std::min(groups, slots);
+    const int64_t live = std::max(gemm_tiles(slots, groups, 16), first);   // (lists as evenly filled as gemm_tiles takes them)
+    const int64_t rows = direct ? first : groups;
+    return Q32Grid{direct ? Q32Grid::DIRECT : Q32Grid::LISTS, live, first, std::max<int64_t>(0, rows * z - live)};
+}
+// An empty workgroup of a fine launch against one of the coarse workgroups that these lines count: it scans the assignments before it
+// leaves, or reads the list's length only.
+inline int64_t q32_empty_weight(const Q32Grid& g) { return g.kind == Q32Grid::LISTS ? 20 : 10; }
+
+// The fine kernels fill the chip where the coarse ones (128 rows of F, 64 of H per workgroup) leave CUs without work.
+//   Up: to 700 coarse workgroups, a list's second and later passes counted twice (they read its weights again).  us, coarse / fine: a quarter of
+//   Mixtral's width, Q4_0, 224 workgroups (up to 40 tokens) 16.8 / 14.6, 448 (100 tokens, two passes) 31.4 / 28.0; three passes 32.8 / 37.2;
+//   Qwen-MoE shape, Q8_0, 44 (one token) 31 / 15, 176 47 / 21, 660 (16 tokens) 54 / 43; Mixtral, Q4_0, 448 (two tokens) 85 / 56, 896 93 / 97.
+//   A one-tile launch some of whose lists may need a second pass stays coarse (Q4_0, 64 tokens 20.8 / 22.6).
+//   Down: to 400 for a dense product (Q8_0 4096 x 4096 64 (16 rows) 21.4 / 11.4, 256 27.8 / 18.6, 448 28.4 / 27.7, 512 28.9 / 30.8), to 340 for
+//   a layer, whose lists are less even (2048 -> 2816, eight experts, top-4, Q4_0, 28 tokens 53.6 / 60.3 at 354, empty ones counted).
+//   Empty workgroups (256 -> 512, 128 experts, top-1, Q4_0, layer: 400 tokens 35.7 / 52.2, 640 tokens 40.8 / 67.1; 1024 -> 2816, 16 experts, top-1,
+//   260 tokens 60.9 / 96.1): at these weights 3 % of the sizes that take a fine kernel lose more than 2 % by it, uncounted 12 %.
+//   The always-on expert: beside the routed launches its passes compete for the chip, and the lines are half as far (4096 -> 1408, 48 experts
+//   with one of 5632, Q8_0: 89 tokens 263 / 279, 113 tokens 272 / 329).
+inline bool q32_up_fine(int64_t F, const Q32Grid& g, int slot_tiles) {
+    if (slot_tiles == 1 && g.live != g.first) return false;
+    return (F / 32 + 3) / 4 * (2 * g.live - g.first) + F / 32 * g.empty / q32_empty_weight(g) <= (g.kind == Q32Grid::ALWAYS_ON ? 350 : 700);
+}
+inline bool q32_down_fine(int64_t H, const Q32Grid& g) {
+    const int64_t line = g.kind == Q32Grid::ROWS ? 400 : g.kind == Q32Grid::ALWAYS_ON ? 200 : 340;
+    return (H / 16 + 3) / 4 * g.live + H / 16 * g.empty / q32_empty_weight(g) <= line;
+}
+
+}  // namespace moe
