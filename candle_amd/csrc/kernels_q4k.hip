@@ -742,9 +742,7 @@ __device__ inline void q4k_up_body(const ExpertParams& p, float (*hbuf)[HBUF_STR
 // the rows in registers / this: 56 tokens 117 / 110 us, 100 tokens 126 / 118, 136 tokens 176 / 163; a quarter of its width, 100 tokens
 // 26.1 / 22.4.  (Q5K unpacks faster sub-block by sub-block than into planes, 108 / 142 here; Q6K measured the same both ways.)
 struct Up2Q4K {
-    typedef Q4KTile Tile;
-    static constexpr int TILE_BYTES = Q4K_TILE_BYTES, LOADS = 3;
-    static constexpr bool kSums = true;
+    static constexpr int LOADS = 3;   // of a weight tile
     struct Scales {
         float d, dmin;
         // the 3-bit digits of the eight scales, one per 16-bit lane (a lane is what the packed multiply can take twice):
@@ -752,10 +750,9 @@ struct Up2Q4K {
         uint32_t hi[4], lo[4];
         v4h mB;
     };
-    static __device__ __forceinline__ Tile load(const uint8_t* tile, int lane) { return load_q4k_tile(tile, lane); }
     // low_half: all ones in lane groups 0 and 1, whose block sums belong to the first four sub-blocks (a mask: a branch would end
     // the loop's basic block)
-    static __device__ __forceinline__ Scales scales(const Tile& w, int g, uint32_t low_half) {
+    static __device__ __forceinline__ Scales scales(const Q4KTile& w, int g, uint32_t low_half) {
         const uint32_t M4 = 0x0f0f0f0fu, M7 = 0x00070007u;
         const uint32_t u0 = w.sc.y, u1 = w.sc.z, u2 = w.sc.w;
         Scales S;
@@ -771,7 +768,7 @@ struct Up2Q4K {
         return S;
     }
     template <int P>
-    static __device__ __forceinline__ void planes(const Tile& w, const Scales& S, int, v4i& hi, v4i& lo) {
+    static __device__ __forceinline__ void planes(const Q4KTile& w, const Scales& S, v4i& hi, v4i& lo) {
         const uint32_t M4 = 0x0f0f0f0fu;
         const uint4& q = P < 2 ? w.q0 : w.q1;
         const uint32_t wx = P & 1 ? q.z : q.x, wy = P & 1 ? q.w : q.y;
@@ -792,9 +789,8 @@ struct Up2Stage {
     _Float16 bs[2][2][2][16][8];         // [buffer][slot tile][half][slot] eight block sums
     float yd[2][64];                     // [buffer][slot] (two copies of the 32)
 };
-template <class FMT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void q4k_up2_kernel(ExpertParams p) {
-    constexpr int NW = 8, RTW = 2, NT = 2 * RTW, RING = 1;
+    constexpr int NW = 8, RTW = 2, NT = 2 * RTW;
     __shared__ __align__(16) uint8_t lds[sizeof(Up2Stage) > 32 * HBUF_STRIDE * 4 ? sizeof(Up2Stage) : 32 * HBUF_STRIDE * 4];
     __shared__ int list_lds[DIRECT_MAX_SLOTS];
     __shared__ int wtot_lds[NW];
@@ -809,18 +805,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const uint8_t* tp[NT];
 #pragma unroll
     for (int j = 0; j < RTW; j++) {
-        tp[j] = gw.w1 + (size_t)(rt0 + j) * FMT::TILE_BYTES;
-        tp[RTW + j] = gw.w3 + (size_t)(rt0 + j) * FMT::TILE_BYTES;
+        tp[j] = gw.w1 + (size_t)(rt0 + j) * Q4K_TILE_BYTES;
+        tp[RTW + j] = gw.w3 + (size_t)(rt0 + j) * Q4K_TILE_BYTES;
     }
-    const size_t sb_stride = (size_t)(F / 16) * FMT::TILE_BYTES;
+    const size_t sb_stride = (size_t)(F / 16) * Q4K_TILE_BYTES;
     if (blockIdx.z > 0 && !p.rb.direct && !p.is_shared) {   // (a later pass: see q4k_up_body)
         const int gi = p.group0 + grp;
         if ((int)blockIdx.z * 32 >= p.rb.offsets[gi + 1] - p.rb.offsets[gi]) return;
     }
-    // first weight tiles go out before anything else; an expert without tokens wastes them
-    typename FMT::Tile ring[RING];
-#pragma unroll
-    for (int j = 0; j < RING; j++) ring[j] = FMT::load(tp[j], lane);
+    // the first weight tile goes out before anything else; an expert without tokens wastes it
+    Q4KTile next = load_q4k_tile(tp[0], lane);
     const GroupSlots gs = group_slots<NW * 64>(p, grp, list_lds, wtot_lds);
     const int tg0 = blockIdx.z * 32;
     if (tg0 >= gs.n) return;
@@ -830,7 +824,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const uint32_t s_src = wave == 0 ? (act_row((lane >> 5) * 16 + r) * (uint32_t)nsb * 16 + (uint32_t)(g & 1) * 8) * 2 : act_row(lane & 31) * (uint32_t)nsb * 4;
     auto stage = [&](int sb, int buf) {
         dma16(p.xq.qs + sb * 256, q_src, lds_address(&L.q[buf][wave >> 2][wave & 3][0]));
-        if (FMT::kSums && wave == 0) dma16(static_cast<const uint8_t*>(p.xq.bsum) + sb * 32, s_src, lds_address(&L.bs[buf][0][0][0][0]));
+        if (wave == 0) dma16(static_cast<const uint8_t*>(p.xq.bsum) + sb * 32, s_src, lds_address(&L.bs[buf][0][0][0][0]));
         if (wave == 1) dma4(p.xq.d + sb, s_src, lds_address(&L.yd[buf][0]));
     };
     stage(0, 0);
@@ -855,19 +849,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < NT; j++) {
-                const typename FMT::Tile w = ring[j % RING];
-                const int jn = (j + RING) % NT;
-                int sbn = sb + (j + RING) / NT;
+                const Q4KTile w = next;
+                const int jn = (j + 1) % NT;
+                int sbn = sb + (j + 1) / NT;
                 sbn = sbn < nsb ? sbn : nsb - 1;
-                ring[j % RING] = FMT::load(tp[jn] + (size_t)sbn * sb_stride, lane);
+                next = load_q4k_tile(tp[jn] + (size_t)sbn * sb_stride, lane);
                 __builtin_amdgcn_sched_barrier(0);
-                const typename FMT::Scales S = FMT::scales(w, g, low_half);
+                const Up2Q4K::Scales S = Up2Q4K::scales(w, g, low_half);
                 const v4i zero = {0, 0, 0, 0};
                 v4i hi[TTL], lo[TTL];
                 auto pair = [&](auto p_tag) {
                     constexpr int P = decltype(p_tag)::value;
                     v4i wh, wl;
-                    FMT::template planes<P>(w, S, g, wh, wl);
+                    Up2Q4K::planes<P>(w, S, wh, wl);
 #pragma unroll
                     for (int tt = 0; tt < TTL; tt++) {
                         const v4i a = *reinterpret_cast<const v4i*>(&L.q[buf][tt][P][lane * 16]);
@@ -881,15 +875,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
                 for (int tt = 0; tt < TTL; tt++) {
                     v4f Dm = {0.f, 0.f, 0.f, 0.f};
-                    if constexpr (FMT::kSums)
-                        Dm = __builtin_amdgcn_mfma_f32_16x16x16f16(*reinterpret_cast<const v4h*>(&L.bs[buf][tt][g >> 1][r][(g & 1) * 4]), S.mB, Dm, 0, 0, 0);
+                    Dm = __builtin_amdgcn_mfma_f32_16x16x16f16(*reinterpret_cast<const v4h*>(&L.bs[buf][tt][g >> 1][r][(g & 1) * 4]), S.mB, Dm, 0, 0, 0);
                     const v4f yd = *reinterpret_cast<const v4f*>(&L.yd[buf][tt * 16 + 4 * g]);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) FMT::result(S, hi[tt][i], lo[tt][i], Dm[i], yd[i], acc[j][tt][i]);
+                    for (int i = 0; i < 4; i++) Up2Q4K::result(S, hi[tt][i], lo[tt][i], Dm[i], yd[i], acc[j][tt][i]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            wait_loads<RING * FMT::LOADS>();   // all but the weight tile requested last: the staged rows have landed
+            wait_loads<Up2Q4K::LOADS>();   // all but the weight tile requested last: the staged rows have landed
             __syncthreads();
         }
         // h = silu(w1 x) * (w3 x), then the 256-row block of every slot is quantised (as in q4k_up_body)
@@ -1056,7 +1049,8 @@ __device__ inline void q4k_down_body(const ExpertParams& p, float (*part)[NTD * 
 
 // One 16-slot tile per pass (small batches): variant 1 (default) 4 waves, 168 VGPRs, three workgroups
 // per CU; variant 0 8 waves, 128 VGPRs.  Two and four tiles per pass (up to 32 / 64 rows per expert
-// without streaming its weights twice) need the registers of a two-waves-per-SIMD launch.
+// without streaming its weights twice) need the registers of a two-waves-per-SIMD launch, except the
+// two-tile up projection (q4k_up2_kernel above), which keeps its activations in LDS.
 DEF_UP(q4k_up_t1_v0, FmtQ4K, 1, 8, 2, 4)
 DEF_UP(q4k_up_t1_v1, FmtQ4K, 1, 4, 2, 3)
 DEF_UP_NARROW(q4k_up_t1_narrow, FmtQ4K, 4, 2, 4)   // 127 registers: a fourth wave per SIMD is free (batch 2: 85 -> 80 us per step)
@@ -1336,7 +1330,7 @@ struct KernelFamily {
 };
 static const KernelFamily* kernel_family(int dt) {
     static const int uv = variant("MOE_UP_VARIANT", 1), dv = variant("MOE_DOWN_VARIANT", 1);
-    static const KernelFamily q4k = {uv == 0 ? q4k_up_t1_v0 : q4k_up_t1_v1, q4k_up_t1_narrow, q4k_up2_kernel<Up2Q4K>, q4k_up_t4,
+    static const KernelFamily q4k = {uv == 0 ? q4k_up_t1_v0 : q4k_up_t1_v1, q4k_up_t1_narrow, q4k_up2_kernel, q4k_up_t4,
                                      dv == 0 ? q4k_down_t1_v0 : q4k_down_t1_v1, q4k_down_t1_narrow, q4k_down_t2, q4k_down_t4,
                                      q4k_down_t1_fine, q4k_down_t2_fine, q4k_down_t4_fine};
     static const KernelFamily q2k = {q2k_up_t1, q2k_up_t1_narrow, q2k_up_t2, nullptr, q2k_down_t1, q2k_down_t1_narrow, q2k_down_t2, nullptr,
