@@ -509,7 +509,7 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
     const int64_t passes = (T + 16 * pl.slot_tiles - 1) / (16 * pl.slot_tiles);
     pl.direct = !pl.tiled && T * L->k <= DIRECT_MAX_SLOTS && T <= DIRECT_MAX_SLOTS && (passes <= 4 || L->E <= 16);
     if (pl.tiled) {
-        const LayerPlan lp = gemm_layer_plan(gemm_format(L->dt), gemm_format(L->dt_down), L->H, L->F, T * L->k, L->E);
+        const LayerPlan lp = gemm_layer_plan(gemm_format(L->dt), gemm_format(L->dt_down), L->H, L->F, T, L->k, L->E);
         pl.tile_slots = lp.tile_slots;
         pl.tiled_down = lp.tiled_down;
     }

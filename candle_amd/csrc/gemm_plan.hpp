@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "../../include/candle_amd_moe.h"
+
 namespace moe {
 
 constexpr int GEMM_MIN_TILE_SLOTS = 64;  // smallest tile of the tiled expert kernels
@@ -92,27 +94,41 @@ inline bool gemm_wide(bool up, int64_t rows, int64_t slots, int64_t groups, int 
 
 // What a tiled launch takes, in us, for choosing between its variants.  A workgroup of eight waves (two per SIMD) needs
 //     0.31 us per super-block and 256 weight rows, times (16-slot operands that hold slots + `unpack`),
-// where `unpack` is what the unpacking of a weight costs beside the product with one operand (gemm_unpack below), and 3 us
+// where `unpack` is what the unpacking of a weight costs beside the product with one operand (GemmFormat below), and 3 us
 // around its K loop; workgroups come in rounds of 32 on the busiest XCD.  Two workgroups of four waves share a CU at 5 % more; one alone
 // takes 0.85 of such a pair's time, which is what makes small grids slow: a wave alone leaves half of its SIMD's cycles
 // empty.  So where a launch would have one of them per CU, the four row groups of a workgroup are given to eight waves, four for
 // each half of K (or two row groups to eight waves, a quarter of K each), and the sums meet in LDS: half (a quarter of) the K
 // steps with every SIMD full, 10 % more per step for the activations fetched per row and 6 us around the loop.
-// Against measurements (Q2_K .. Q6_K, 4096 x 4096, 1024 x 4096, 14336 x 4096 and 4096 x 14336 at 96 to 4096 rows; Mixtral's shape and
-// a quarter of it at 137 to 3000 tokens) the variant chosen by this is 1 % off the best one on average.  One part / the
+// Against measurements (2043 dense products of 96 to 3000 rows, 3378 layers of 4 to 160 experts with 34 to 500 rows each, the five
+// formats, even and skewed lists, every variant timed at each) the choices by this file are 1.7 % off the best variant on average, 5 % of
+// the layers and 1.4 % of the products 3 % or more slower than by fixed lines (tiled down projections from 64 rows per expert on, 128
+// slots from 72; tiled products from 192 workgroups on, 128 slots from 512; one part), and the mean 7.5 % and 6 % faster.  One part / the
 // choice: Q4_K 4096 x 4096 at 384 rows 36.8 / 31.6, at 777 51.2 / 45.4, 4096 x 14336 at 512 rows 107 / 90, 14336 x 4096 at 128
 // 47 / 32; Q6_K 4096 x 4096 at 777 58.1 / 49.1; at a full chip it costs: Q4_K 4096 x 4096 at 4096 rows 161 / 181.
 struct GemmPlan {
     int parts;    // parts K is cut into: 1 (workgroups as gemm_wide says), 2 (128-row workgroups), 4 (64-row ones, tiles of 64 slots)
     double us;
 };
+// What a workgroup of 64 rows and a pass of the streaming down kernels takes, in us times the CUs: around its K loop, per super-block, and
+// one that finds no slots; dense: of the dense products' rate below.
+struct StreamCost { double wg, step, empty, dense; };
 // format traits of the tiled kernel: unpack, in operands; one_operand: launches in tiles of 64 slots have one 16-row weight
 // operand per wave; crowded: with 128 slots and the two accumulator sets of a split the registers overflow beyond 96 slots
 struct GemmFormat {
     double unpack;
     bool one_operand, crowded;
     bool four_tiles;   // the streaming kernels carry 64 slots per pass, not 32
+    StreamCost stream;
 };
+// (the unpacking measured beside the product with one 16-slot operand)
+inline GemmFormat gemm_format(int dt) {
+    const bool one_operand = dt == MOE_GGML_Q3K || dt == MOE_GGML_Q5K || dt == MOE_GGML_Q6K;
+    const StreamCost s = dt == MOE_GGML_Q2K ? StreamCost{2.6, 0.44, 0.18, 0.78} : dt == MOE_GGML_Q3K ? StreamCost{2.0, 0.62, 0.19, 1.0}
+                       : dt == MOE_GGML_Q4K ? StreamCost{5.0, 0.78, 0.5, 1.0}  : dt == MOE_GGML_Q5K ? StreamCost{2.4, 0.63, 0.19, 1.0}
+                                                                               : StreamCost{2.3, 0.71, 0.185, 1.0};
+    return GemmFormat{one_operand ? 5.0 : 2.5, one_operand, dt == MOE_GGML_Q5K, dt == MOE_GGML_Q4K, s};
+}
 inline GemmPlan gemm_plan(const GemmFormat& f, bool up, int64_t rows, int64_t k, int64_t slots, int64_t groups, int tile_slots, int64_t max_tiles) {
     const int64_t nsb = k / 256, tiles = std::min(gemm_tiles(slots, groups, tile_slots), max_tiles);
     // 16-slot operands of a tile: of the longest of a dense product, on average over lists
@@ -140,44 +156,59 @@ inline GemmPlan gemm_plan(const GemmFormat& f, bool up, int64_t rows, int64_t k,
     }
     return best;
 }
-// The streaming down kernels, in us.  They give a workgroup 64 rows and a pass of 64 slots (four_tiles: Q4K) in 1.07 us per
-// super-block, in rounds of a workgroup per CU, or passes of 32 slots, where only the number of (16 rows x 32 slots) products
-// counts, 0.83 ns each.
-inline double streamed_us(bool four_tiles, int64_t rows, int64_t k, int64_t slots, int64_t groups) {
-    const int64_t nsb = k / 256, passes = gemm_tiles(slots, groups, four_tiles ? 64 : 32);
-    if (!four_tiles) return 2 + 0.83e-3 * (double)(rows / 16 * passes * nsb);
+// The streaming down kernels, in us.  They give a workgroup 64 rows and a pass of 64 slots (four_tiles: Q4K) or 32.
+//   Over expert lists the grid holds a pass for every 64 (32) tokens there could be in a list, most of them empty, and workgroups end at
+//   different times: no rounds.  Few super-blocks cost little more than one (F = 256, where tiled and streamed looked alike without the
+//   two constants: 3840 -> 256, 34 experts, Q4_K, 3089 tokens, step, tiled / streamed 195 / 511; 768 -> 256, 42 experts, 5591 tokens 82 / 191).
+inline double streamed_lists_us(const GemmFormat& f, int64_t rows, int64_t k, int64_t tokens, int64_t slots, int64_t groups) {
+    const int64_t nsb = k / 256, pass = f.four_tiles ? 64 : 32;
+    const int64_t live = rows / 64 * gemm_tiles(slots, groups, (int)pass), all = rows / 64 * groups * ((tokens + pass - 1) / pass);
+    return 4 + std::max(1.0, (double)live / 256) * (f.stream.wg + f.stream.step * (double)nsb) * (live <= 64 ? 0.65 : 1.0) +
+           f.stream.empty * (double)std::max<int64_t>(0, all - live) / 256;
+}
+//   Dense products: rounds of a workgroup per CU, 1.07 us per super-block (Q4K), or only the number of (16 rows x 32 slots) products counts,
+//   0.83 ns each (Q2K 0.65: 1024 x 14336 at 480 rows 49, four parts of 64 slots 61).
+inline double streamed_us(const GemmFormat& f, int64_t rows, int64_t k, int64_t slots) {
+    const int64_t nsb = k / 256, passes = gemm_tiles(slots, 1, f.four_tiles ? 64 : 32);
+    if (!f.four_tiles) return 2 + 0.83e-3 * f.stream.dense * (double)(rows / 16 * passes) * (0.95 * (double)nsb + 1);
     const int64_t wgs = rows / 64 * passes;
-    return 2 + (double)((wgs + 255) / 256 * nsb) * (wgs <= 64 ? 0.7 : 1.07);
+    return 2 + (double)((wgs + 255) / 256) * (1.07 * (double)nsb + 0.5) * (wgs <= 64 ? 0.65 : 1.0);
 }
 // A routed layer (w1 and w3 of F rows each over H, w2 of H rows over F): the slots per tile, 64 or 128, by the sum of its two
 // launches, and whether the down projection is tiled as well.  (Mixtral shape, us per step, 64 / 128: Q4_K 40 rows per expert
 // 282 / 281, 50 rows 308 / 302, 60 rows 388 / 323, 75 rows 437 / 354; a quarter of its width: 75 rows 60 / 69, 125 rows 76 / 92, 250 rows
 // 126 / 115.  The down launch alone, streamed / tiled: Q4_K 25 rows 69 / 69, 34 rows 99 / 83, 50 rows 112 / 93; Q6_K 34 rows 145 / 105,
 // 50 rows 173 / 118; a quarter of the width Q4_K 35 rows 20 / 17, Q6_K 35 rows 19 / 21, 75 rows 27 / 23.)
+// The costs know the mean of the lists only.  What that leaves uncertain goes to the side where the loss is small: 128 slots below 40 rows
+// per expert where they promise a tenth (1280 -> 3584, 15 experts, Q5_K, 562 tokens, Zipf loads, 64 / 128 90 / 117), and no streaming
+// beyond 200, where the longest list decides (256 -> 7168, 16 experts, top-1, Q4_K, 4857 tokens, Zipf loads, tiled / streamed 199 / 331).
 struct LayerPlan {
     int tile_slots;
     bool tiled_down;
 };
-inline LayerPlan gemm_layer_plan(const GemmFormat& f_up, const GemmFormat& f_down, int64_t H, int64_t F, int64_t slots, int64_t groups) {
-    const double streamed = streamed_us(f_down.four_tiles, H, F, slots, groups);
+inline LayerPlan gemm_layer_plan(const GemmFormat& f_up, const GemmFormat& f_down, int64_t H, int64_t F, int64_t tokens, int64_t top_k, int64_t groups) {
+    const int64_t slots = tokens * top_k;
+    const double streamed = slots > 200 * groups ? 1e30 : streamed_lists_us(f_down, H, F, tokens, slots, groups);
     LayerPlan best{64, false};
     double us = 0;
     for (int tile = 64; tile <= 128; tile *= 2) {
         const int64_t max_tiles = max_gemm_tiles(slots, groups + 1, tile);
         const double down = gemm_plan(f_down, false, H, F, slots, groups, tile, max_tiles).us;
         const double t = gemm_plan(f_up, true, 2 * F, H, slots, groups, tile, max_tiles).us + std::min(down, streamed);
-        if (tile == 64 || t <= us) { best = LayerPlan{tile, down <= streamed}; us = t; }
+        if (tile == 64 || t <= us * (slots < 40 * groups ? 0.9 : 1.0)) { best = LayerPlan{tile, down <= streamed}; us = t; }
     }
     return best;
 }
 // Slots per tile of a dense product of m rows with an [n, k] matrix, or 0 where the streaming kernels are faster.  (us, streamed /
 // tiled: Q4_K 4096 x 4096 at 256 rows 24.9 / 25.0, 320 36 / 31; 1024 x 4096 at 256 18.8 / 23.1, 512 25.6 / 25.3; 14336 x 4096 at
-// 96 38.7 / 29.4; Q6_K 4096 x 4096 at 128 rows 19.7 / 24.4, 192 28.6 / 25.3; 14336 x 4096 at 96 41.4 / 35.8.)
+// 96 38.7 / 29.4; Q6_K 4096 x 4096 at 128 rows 19.7 / 24.4, 192 28.6 / 25.3; 14336 x 4096 at 96 41.4 / 35.8; Q4_K 4096 x 512 at 440 18.3 / 10.7.)
+// On a chip that 128-slot tiles fill twice they are the better ones where the costs are close (Q4_K, 64 / 128: 4096 x 4096 at 2059 rows
+// 104 / 92, 14336 x 4096 at 572 112 / 98).
 inline int gemm_dense_tile(const GemmFormat& f, int64_t n, int64_t k, int64_t m) {
     if (n % 128 || m < 96) return 0;
-    const double us64 = gemm_plan(f, false, n, k, m, 1, 64, max_gemm_tiles(m, 2, 64)).us;
+    const double us64 = gemm_plan(f, false, n, k, m, 1, 64, max_gemm_tiles(m, 2, 64)).us / (n / 128 * ((m + 127) / 128) >= 512 ? 0.95 : 1.0);
     const double us128 = gemm_plan(f, false, n, k, m, 1, 128, max_gemm_tiles(m, 2, 128)).us;
-    return streamed_us(f.four_tiles, n, k, m, 1) <= std::min(us64, us128) ? 0 : us128 <= us64 ? 128 : 64;
+    return streamed_us(f, n, k, m) <= std::min(us64, us128) ? 0 : us128 <= us64 ? 128 : 64;
 }
 
 }  // namespace moe

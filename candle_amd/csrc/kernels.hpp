@@ -134,11 +134,6 @@ hipError_t launch_expert_down(const ExpertParams& p, hipStream_t s);
 // caller re-quantises it), down writes yw.
 bool q4k_gemm_up_format(int dt);
 bool q4k_gemm_down_format(int dt);
-// What the plans of gemm_plan.hpp need to know of a K-quant: its unpacking measured beside the product with one 16-slot operand.
-inline GemmFormat gemm_format(int dt) {
-    const bool one_operand = dt == MOE_GGML_Q3K || dt == MOE_GGML_Q5K || dt == MOE_GGML_Q6K;
-    return GemmFormat{one_operand ? 5.0 : 2.5, one_operand, dt == MOE_GGML_Q5K, dt == MOE_GGML_Q4K};
-}
 // Dense matrix [n, k] (device layout) times m <= 4 rows of f32 in one launch (the rows are quantised in the kernel).
 struct FusedRows {
     const float* x = nullptr;          // [m, k] rows ...
