@@ -261,6 +261,8 @@ Switches& switches() {
         g_sw.slot_tiles = (int)num("MOE_SLOT_TILES", 0);
         g_sw.narrow = (int)num("MOE_NARROW", -1);
         g_sw.fused_rows = (int)num("MOE_FUSED_ROWS", 0);
+        g_sw.tiled_down = (int)num("MOE_TILED_DOWN", -1);
+        g_sw.k_parts = (int)num("MOE_K_PARTS", 0);
     });
     return g_sw;
 }
@@ -514,6 +516,7 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
         pl.tiled_down = lp.tiled_down;
     }
     if (sw.tile_slots == 64 || sw.tile_slots == 128) pl.tile_slots = sw.tile_slots;
+    if (pl.tiled && sw.tiled_down >= 0) pl.tiled_down = sw.tiled_down > 0;
     // Top-2 routing with nothing else to add to a token's result (no shared expert, no residual): the streaming down
     // kernels add their two terms per token straight into the output, which the front kernel clears, and no combine
     // pass runs (a + b is the same float in either order; with three or more terms the order would matter).  Batches
@@ -639,6 +642,7 @@ static int enqueue_forward(moe_layer* L, const ForwardPlan& pl, const Workspace&
     ep.y_acc = pl.accumulate ? d_y : nullptr;
     ep.max_rows = T;
     ep.slot_tiles = pl.slot_tiles;
+    ep.k_parts = switches().k_parts;
     // The always-on expert reads the quantised activations and writes its own slots of yw: independent of the routed
     // experts until the combine pass, so its kernels go to the side stream and fill the CUs the routed launches leave idle
     // (the timed entry keeps one stream: its stage marks would mean nothing otherwise).
@@ -1226,7 +1230,9 @@ static int enqueue_qlinear(moe_qlinear* Q, const float* d_x, int64_t m, float* d
         if (int rc = Q->order.enter(s)) return rc;
     // K-quants: streamed, or tiled with the tile that the costs of gemm_plan.hpp say
     const int64_t row_blocks = Q->n / 128;
-    const int k_tile = !switches().no_gemm && q4k_gemm_down_format(Q->dt) ? gemm_dense_tile(gemm_format(Q->dt), Q->n, Q->k, m) : 0;
+    int k_tile = !switches().no_gemm && q4k_gemm_down_format(Q->dt) ? gemm_dense_tile(gemm_format(Q->dt), Q->n, Q->k, m) : 0;
+    if (switches().tiled_down >= 0 && q4k_gemm_down_format(Q->dt) && Q->n % 128 == 0)
+        k_tile = switches().tiled_down == 0 ? 0 : switches().tile_slots == 128 ? 128 : 64;
     const bool tiled = k_tile != 0;
     const int tile_slots = tiled ? k_tile : 64;
     // Q8_0 / Q4_0 / Q5_0 matrices: the tiled kernel of the 32-element formats (64-row tiles of the one group, no tile list)
@@ -1248,6 +1254,7 @@ static int enqueue_qlinear(moe_qlinear* Q, const float* d_x, int64_t m, float* d
     ep.groups = Q->group.as<GroupWeights>();
     ep.rb = rb; ep.hq = xq; ep.slot_origin = 0; ep.yw = d_y;
     ep.max_rows = m; ep.n_slots = m; ep.slot_tiles = m > 32 ? 4 : m > 16 ? 2 : 1;
+    ep.k_parts = switches().k_parts;
     if (tiled) {
         MOE_HIP_CHECK(launch_q4k_gemm_down(ep, s));
     } else if (tiled32) {
@@ -1412,6 +1419,8 @@ extern "C" int moe_debug_set_switch(const char* name, int64_t value) {
     else if (n == "fused_rows") sw.fused_rows = (int)value;
     else if (n == "front_split") sw.front_split = (int)value;
     else if (n == "dispatch_one") sw.dispatch_one = (int)value;
+    else if (n == "tiled_down") sw.tiled_down = (int)value;
+    else if (n == "k_parts") sw.k_parts = (int)value;
     else return fail(MOE_E_INVALID, "moe_debug_set_switch: unknown switch '" + n + "'");
     return MOE_OK;
 }

@@ -19,6 +19,8 @@ struct Switches {
     int slot_tiles = 0;               // MOE_SLOT_TILES: 16-slot tiles per streaming pass (0 = by batch size)
     int narrow = -1;                  // MOE_NARROW: 0 | 1 (-1 = by batch size)
     int fused_rows = 0;               // MOE_FUSED_ROWS: dense products of a few rows in one launch: 1 = never, 2 = whenever possible (0 = by size)
+    int tiled_down = -1;              // MOE_TILED_DOWN: K-quants, w2 of a layer whose up projection is tiled and dense products: 0 streamed | 1 tiled, of tile_slots slots (-1 = by cost)
+    int k_parts = 0;                  // MOE_K_PARTS: tiled K-quant down launches, parts of K: 1 | 2 | 4 (tiles of 64) (0 = by cost)
 };
 Switches& switches();
 
@@ -123,6 +125,7 @@ struct ExpertParams {
     int down_interleaved = 0;   // down projection: wave w of a workgroup takes super-blocks w, w + NW, ... instead of a contiguous range
     float* hbuf = nullptr;          // tiled path only: f32 intermediate [slots, F] before re-quantisation
     int64_t n_slots = 0;            // tiled path only: total slots (bounds the tile grid)
+    int k_parts = 0;                // tiled down launches: parts K is cut into (testing aid; 0: as gemm_plan says)
 };
 // h = silu(W1 x) * (W3 x), quantised to the activation format, for every slot of every group.
 hipError_t launch_expert_up(const ExpertParams& p, hipStream_t s);

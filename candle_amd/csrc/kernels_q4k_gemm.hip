@@ -29,14 +29,14 @@
 // fetched nor multiplied (the K loop exists for each number of them).
 // Down launches of the formats that unpack longest in tiles of 64 slots run one operand per wave at four waves per SIMD
 // (launch_gemm).  Registers: 164 to 254 with two operands (Q5K at 128 slots: 256, one to three of them spilled outside the K
-// loop), 122 to 126 with one.
+// loop, ten with K split, Q4K split one), 122 to 126 with one.
 //
 // Where a launch would have no more than one workgroup of four waves per CU (a down projection of some hundred tokens, dense products
 // of a few hundred rows), a wave alone on its SIMD leaves it idle for two fifths of the time, and nothing else is there to run.
 // There the workgroup has eight waves for the same rows, four for each half of K with LDS buffers of their own (KS = 2; KS = 4:
 // two waves for each quarter, 64 rows), whose sums meet in LDS at the end.  Down launch, Mixtral shape: Q4_K 200 tokens 112 -> 93 us,
 // 301 tokens 128 -> 111; Q6_K 301 tokens 153 -> 135.  The rule and the dense products' times: gemm_plan.hpp.  On a full chip the split
-// costs (Q4_K 4096 x 4096 at 4096 rows 161 -> 181): there the chip's power is the bound, the clock falls from 2.2 to 1.7 GHz.
+// costs (Q4_K 4096 x 4096 at 4096 rows 161 -> 181).
 //
 // Q6K weights (the w2 of mixed files) take the same kernel for the down projection.  BlockQ6K::vec_dot
 // (k_quants.rs:1613-1671) is d * y.d * sum_j sc_j * ((code_j - 32) . q8_j) with an i8 scale per 16 elements; the
@@ -613,8 +613,8 @@ static void launch_gemm(ExpertParams& p, hipStream_t s) {
     };
     // K split over the waves of a workgroup where the grid would leave SIMDs with one wave or none (gemm_plan)
     if constexpr (MODE == 1) {
-        const int parts = gemm_plan(gemm_format(FMT), false, rows, p.F, p.n_slots, p.n_groups, p.rb.tile_slots, tiles).parts;
-        if (parts == 4) return launch(q4k_gemm_kernel<FMT, 1, 4, 8, 2, 4>, 8, 64);
+        const int parts = p.k_parts ? p.k_parts : gemm_plan(gemm_format(FMT), false, rows, p.F, p.n_slots, p.n_groups, p.rb.tile_slots, tiles).parts;
+        if (parts == 4 && tiles64) return launch(q4k_gemm_kernel<FMT, 1, 4, 8, 2, 4>, 8, 64);
         if (parts == 2) return tiles64 ? launch(q4k_gemm_kernel<FMT, 1, 4, 8, 2, 2>, 8, 128) : launch(q4k_gemm_kernel<FMT, 1, 8, 8, 2, 2>, 8, 128);
     }
     const bool wide = !(one_operand && tiles64) && gemm_wide(MODE == 0, rows, p.n_slots, p.n_groups, p.rb.tile_slots, tiles);

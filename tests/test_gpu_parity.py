@@ -324,9 +324,8 @@ def test_block_q4k_shared_expert_slot_tiles(T):
 
 def test_block_q4k_tile_sizes_and_paths():
     # two slot tiles per streamed pass with a second pass for lists beyond 32 rows (T = 104, 130); from 35 rows per
-    # expert the tiled kernel for the up projection with the down projection still streamed, four slot tiles per pass
-    # (T = 140, 150, 160, 200, 250), from 65 rows for both: 64-slot tiles (T = 270) up to ~72 rows per expert,
-    # 128 beyond (T = 300, 400, 600)
+    # expert the tiled kernels for both projections, tiles of 64 slots, w2 in four parts of K (tiles of 128 slots and the
+    # other splits: test_gpu_k_split.py)
     ref, gpu = make_pair(512, 1024, 8, 2, O.Q4K, seed=1)
     for T in (104, 130, 140, 150, 160, 200, 250, 270, 300, 400, 600):
         check_block(ref, gpu, T)
@@ -339,8 +338,8 @@ def test_block_q6k_and_mixed_down_dtype(dt, dt_down):
     # all-Q6K and all-Q5K experts, the Q4_K_M arrangement (Q4K gate / up with Q6K down), its reverse, and
     # the Q5_K_M arrangement (Q5K with Q6K down).
     # T = 1, 3: narrow workgroups; 8, 33: one and two slot tiles per pass; 70: dispatched lists;
-    # 200: a K-quant up projection switches to the tiled kernel; 300, 500: so does such a down projection
-    # behind it (64-slot and 128-slot tiles)
+    # 200: a K-quant up projection switches to the tiled kernel; 500: so does every such down projection
+    # behind it (tiles of 64 slots, four parts of K)
     ref, gpu = make_pair(512, 1024, 8, 2, dt, seed=12, dt_down=dt_down)
     for T in (1, 3, 8, 33, 70, 200, 300, 500):
         check_block(ref, gpu, T, tol=block_tol(O.Q4K, 1024))

@@ -61,9 +61,10 @@ def test_every_number_of_live_operands_in_tiles_of_128_rows(dt, n, k):
     check(dt, n, k, (130, 150, 176, 192, 200, 220, 239, 256), simd=True)
 
 
-# Layers of eight experts, top-2, whose lists end in different operands of a tile.  Up projection: tiles of 64 slots
-# (200, 240, 270 tokens) and of 128, four-wave workgroups (F = 512, 768) and eight-wave ones (F = 2048 from 600 tokens on).  Down:
-# 64 slots (270), 128; four waves (H = 768) and eight (H = 4096).
+# Layers of eight experts, top-2, whose lists end in different operands of a tile.  Up projection: tiles of 64 slots and of 128,
+# four-wave workgroups (F = 512, 768) and eight-wave ones (F = 2048).  Down, as the costs have it (tests/test_gemm_split_plan_cpu.py):
+# one part (F = 512, 768; eight waves at H = 4096), two parts of 128 slots (F = 2048), four of 64 (F = 1024; Q3K streamed).  Every down
+# kernel at every size: test_gpu_k_split.py.
 # The bar is that of any narrow K-quant layer: an f32 sum in another order moves a value of the intermediate by one quantisation
 # step now and then, which weighs sqrt(14336 / F) times what it does at F = 14336 (there 2e-3 max and 2e-4 rms).  A row beyond
 # it has to be within it once such steps, four at most, are taken out (FlipExplainer).
