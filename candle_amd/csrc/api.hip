@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "kernels.hpp"
+#include "q32_plan.hpp"
 
 namespace moe {
 
@@ -507,7 +508,9 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
     // small batches: slots are numbered t*k + r and no dispatch pass runs; every workgroup then finds its expert's slots
     // by scanning the assignments, and the grid holds a pass for every 16 * slot_tiles tokens there could be in a list.
     // With many experts most of those passes are empty: beyond four of them the dispatch pass is worth its 5 us (its
-    // lists let an empty pass leave at once; 128 experts, 512 tokens: 386 -> 303 us).
+    // lists let an empty pass leave at once; 128 experts, 512 tokens: 386 -> 303 us.  32-element formats, more than 16 experts, without /
+    // with the pass, mean over random sizes of 9 to 16 rows per expert, one tile per pass: four passes 0.96, five 0.98, six 1.00, seven 1.02, eight and
+    // nine 1.03 to 1.07, eleven 1.13.)
     const int64_t passes = (T + 16 * pl.slot_tiles - 1) / (16 * pl.slot_tiles);
     pl.direct = !pl.tiled && T * L->k <= DIRECT_MAX_SLOTS && T <= DIRECT_MAX_SLOTS && (passes <= 4 || L->E <= 16);
     if (pl.tiled) {
@@ -538,14 +541,8 @@ static ForwardPlan plan_forward(const moe_layer* L, int64_t T) {
         // at three, 115 / 112 at four; 64 Q4_K experts top-6 with Fs = 3072: 63 / 70, 65 / 75, 67 / 76, 70 / 81)
         pl.shared_rows = can && (sw.fused_rows == 2 || T <= (kq ? 4 : 3));
     }
-    // Q8_0 / Q4_0 / Q5_0 layers whose slots are grouped by expert (more than DIRECT_MAX_SLOTS assignments): the tiled
-    // kernels of kernels_q32.hip read an expert's weights once for up to 64 of its slots
-    // (Many experts: from 13 rows per expert on -- the lists are short of a tile, but a streaming launch over a measured list holds a
-    // workgroup for every pass a list could need, most of them empty.  Streamed / tiled, us, Q8_0: Qwen-MoE shape 120 tokens, 8 rows per
-    // expert, 191 / 218, 170 tokens 204 / 202, 220 tokens 250 / 200, 300 tokens 243 / 220; without its always-on expert 170 tokens
-    // 145 / 159, 220 tokens 175 / 155; 32 experts of 4096 x 4096, top-2, 240 tokens, 15 rows, 433 / 345, 300 tokens 373 / 379; 128 experts
-    // of 1024 x 512, top-8, 180 tokens, 11 rows, 92 / 82.  Up to 16 experts: Mixtral shape, Q4_0, 60 tokens, 15 rows, 219 / 247.)
-    pl.tiled32 = !sw.no_gemm && !pl.direct && q8_0_gemm_usable(L->dt, L->dt_down, L->H, L->F) && T * L->k > (L->E > 16 ? 13 : 20) * L->E;
+    // 32-element layers whose slots a dispatch pass has grouped by expert: q32_plan.hpp
+    pl.tiled32 = !sw.no_gemm && !pl.direct && q8_0_gemm_usable(L->dt, L->dt_down, L->H, L->F) && q32_tiled(T, L->k, L->E);
     if (pl.tiled32) pl.tile_slots = 64;
     return pl;
 }

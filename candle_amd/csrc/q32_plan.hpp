@@ -1,5 +1,5 @@
-// Which kernels a streaming launch of the 32-element formats takes: workgroups of a quarter of the rows ("fine") or whole ones.
-// Plain C++: no HIP types.
+// Which kernels a layer of the 32-element formats takes: tiled or streaming ones, and of the latter workgroups of a quarter of the
+// rows ("fine") or whole ones.  Plain C++: no HIP types.
 //
 // The lines are those of 10962 measured (layer, tokens) pairs: 1160 random layers of 4 to 256 experts (H 256 .. 4096, F 128 .. 8192, top-1
 // to top-10, the five formats, with and without an always-on expert), 0.05 to 33 rows per expert, every variant timed at each.
@@ -10,6 +10,20 @@
 #include "gemm_plan.hpp"
 
 namespace moe {
+
+// Tiled kernels (an expert's weights are read once for up to 64 of its slots) or streaming ones, for layers whose slots a dispatch pass
+// has grouped by expert: from 20 rows per expert on, and below as far as the streaming grids hold passes for lists that are not there
+// -- one for every 16 tokens and expert, most of them empty: from 17 - passes / 5 rows on.  Experts' number and size alone say little.
+//   One tile per pass / tiled, mean time over 4167 random sizes of more than 16 experts: 9 to 13 rows per expert and 8 to 11 passes 0.89,
+//   40 to 79 passes 1.08, more 1.38; 16 to 20 rows, 8 to 11 passes 0.96, 12 to 39 1.03, more 1.16 to 1.41.  us, streamed / tiled, Q8_0: Qwen-MoE
+//   shape 120 tokens, 8 rows per expert, 191 / 218, 220 tokens 250 / 200; Q5_0, 384 -> 3200, 248 experts, top-1, 2772 tokens, 11 rows, 667 / 377.  (Where
+//   it is wrong: 640 -> 2048, 214 experts, top-8, 320 tokens, 12 rows, 243 / 180; 1536 -> 640, 44 experts, 18 rows, 9 passes 80 / 104.)
+//   A line at 13 rows for every number of passes was 3 % or more slower than one at 20 in 3.9 % of those sizes, this one is in 2.8 %.
+//   (Up to 16 experts no dispatch pass runs below 64 rows per expert.)
+inline bool q32_tiled(int64_t T, int64_t k, int64_t E) {
+    const int64_t slots = T * k, passes = (T + 15) / 16;
+    return slots > 20 * E || (slots > 6 * E && 5 * slots + passes * E >= 85 * E);
+}
 
 // What a streaming launch's grid holds, in passes of 16 slots.
 struct Q32Grid {

@@ -15,6 +15,7 @@ extern "C" int fine(int64_t H, int64_t F, int64_t groups, int64_t k, int direct,
     const Q32Grid g = q32_grid(T, k, groups, direct != 0, always_on != 0);
     return q32_up_fine(F, g, tiles) + 2 * q32_down_fine(H, g);
 }
+extern "C" int tiled32(int64_t T, int64_t k, int64_t E) { return q32_tiled(T, k, E); }
 // A tiled K-quant launch over `groups` lists: 1000 * tile + 10 * parts of K + (eight waves with rows of their own)
 static int kernel(int dt, bool up, int64_t rows, int64_t k, int64_t slots, int64_t groups, int tile) {
     const GemmFormat f = gemm_format(dt);
@@ -53,6 +54,7 @@ def load():
     shutil.rmtree(d)
     i64, i = ctypes.c_int64, ctypes.c_int
     lib.fine.argtypes = [i64, i64, i64, i64, i, i, i, i64]
+    lib.tiled32.argtypes = [i64, i64, i64]
     lib.dense_kernel.argtypes = [i, i64, i64, i64]
     lib.up_kernel.argtypes = lib.down_kernel.argtypes = [i, i, i64, i64, i64, i64, i64]
     return lib

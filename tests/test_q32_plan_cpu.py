@@ -32,3 +32,22 @@ def plan():
 ])
 def test_fine_kernels(plan, args, want):
     assert plan.fine(*args) == want
+
+
+# (tokens, top-k, experts), slots grouped by a dispatch pass.  us, streamed / tiled
+@pytest.mark.parametrize("args,want", [
+    ((120, 4, 60), 0),       # 8 rows per expert: 191 / 218
+    ((170, 4, 60), 0),       # 11: 145 / 159
+    ((220, 4, 60), 1),       # 15: 250 / 200
+    ((320, 8, 214), 0),      # 12 rows, 20 passes: even over layers, 243 / 180 here
+    ((1970, 1, 206), 1),     # 9.6 rows, 124 passes: 171 / 114
+    ((1250, 1, 206), 1),     # 6.1 rows, 79 passes: means 1.05
+    ((1200, 1, 206), 0),
+    ((2772, 1, 248), 1),     # 667 / 377
+    ((133, 6, 44), 1),       # 18 rows, 9 passes
+    ((350, 2, 50), 1),       # 14 rows, 22 passes
+    ((21, 64, 64), 1),       # above 20 rows
+    ((150, 3, 32), 0),       # 14 rows, 10 passes
+])
+def test_tiled_kernels(plan, args, want):
+    assert plan.tiled32(*args) == want
