@@ -885,7 +885,7 @@ static hipError_t launch_q32_up_t(const ExpertParams& p, hipStream_t s) {
     const int wpb = Q32_THREADS / 64;
     const int n_pairs = p.F / 32;
     dim3 grid((unsigned)((n_pairs + wpb - 1) / wpb), (unsigned)p.n_groups, (unsigned)((p.max_rows + tt * 16 - 1) / (tt * 16)));
-    if (stream && q32_up_fine(p.F, q32_grid(p), tt)) {
+    if (stream && q32_up_fine(p.F, q32_grid(p))) {
         ExpertParams q = p;
         const dim3 fine = q32_fine_grid(q, n_pairs);
         hipLaunchKernelGGL((q32s_up_fine_kernel<DT, 2>), fine, dim3(Q32_THREADS), 0, s, q);

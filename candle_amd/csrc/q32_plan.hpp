@@ -40,28 +40,26 @@ inline Q32Grid q32_grid(int64_t T, int64_t k, int64_t groups, bool direct, bool 
     const int64_t rows = direct ? first : groups;
     return Q32Grid{direct ? Q32Grid::DIRECT : Q32Grid::LISTS, live, first, std::max<int64_t>(0, rows * z - live)};
 }
-// An empty workgroup of a fine launch against one of the coarse workgroups that these lines count: it scans the assignments before it
-// leaves, or reads the list's length only.
-inline int64_t q32_empty_weight(const Q32Grid& g) { return g.kind == Q32Grid::LISTS ? 20 : 10; }
-
-// The fine kernels fill the chip where the coarse ones (128 rows of F, 64 of H per workgroup) leave CUs without work.
-//   Up: to 700 coarse workgroups, a list's second and later passes counted twice (they read its weights again).  us, coarse / fine: a quarter of
-//   Mixtral's width, Q4_0, 224 workgroups (up to 40 tokens) 16.8 / 14.6, 448 (100 tokens, two passes) 31.4 / 28.0; three passes 32.8 / 37.2;
-//   Qwen-MoE shape, Q8_0, 44 (one token) 31 / 15, 176 47 / 21, 660 (16 tokens) 54 / 43; Mixtral, Q4_0, 448 (two tokens) 85 / 56, 896 93 / 97.
-//   A one-tile launch some of whose lists may need a second pass stays coarse (Q4_0, 64 tokens 20.8 / 22.6).
-//   Down: to 400 for a dense product (Q8_0 4096 x 4096 64 (16 rows) 21.4 / 11.4, 256 27.8 / 18.6, 448 28.4 / 27.7, 512 28.9 / 30.8), to 340 for
-//   a layer, whose lists are less even (2048 -> 2816, eight experts, top-4, Q4_0, 28 tokens 53.6 / 60.3 at 354, empty ones counted).
-//   Empty workgroups (256 -> 512, 128 experts, top-1, Q4_0, layer: 400 tokens 35.7 / 52.2, 640 tokens 40.8 / 67.1; 1024 -> 2816, 16 experts, top-1,
-//   260 tokens 60.9 / 96.1): at these weights 3 % of the sizes that take a fine kernel lose more than 2 % by it, uncounted 12 %.
-//   The always-on expert: beside the routed launches its passes compete for the chip, and the lines are half as far (4096 -> 1408, 48 experts
-//   with one of 5632, Q8_0: 89 tokens 263 / 279, 113 tokens 272 / 329).
-inline bool q32_up_fine(int64_t F, const Q32Grid& g, int slot_tiles) {
-    if (slot_tiles == 1 && g.live != g.first) return false;
-    return (F / 32 + 3) / 4 * (2 * g.live - g.first) + F / 32 * g.empty / q32_empty_weight(g) <= (g.kind == Q32Grid::ALWAYS_ON ? 350 : 700);
+// The fine kernels fill the chip where the coarse ones (128 rows of F, 64 of H per workgroup) leave CUs without work.  Counted in coarse
+// workgroups of passes that find slots; the empty ones of a fine launch at a 40th (up), a 20th (down) of a coarse one each where lists
+// are found by scanning the assignments, at a 30th where a dispatch pass has measured them.
+//   Up: to 800, a list's second and later passes counted 1.3 times (they read its weights again).  us, coarse / fine: a quarter of
+//   Mixtral's width, Q4_0, 224 workgroups (up to 40 tokens) 16.8 / 14.6, 448 (100 tokens, two passes) 31.4 / 28.0; Qwen-MoE shape, Q8_0, 44
+//   (one token) 31 / 15, 176 47 / 21, 660 (16 tokens) 54 / 43; Mixtral, Q4_0, 448 (two tokens) 85 / 56, 896 93 / 97.
+//   Down: to 400.  Dense, Q8_0 4096 x 4096, 64 (16 rows) 21.4 / 11.4, 256 27.8 / 18.6, 448 28.4 / 27.7, 512 28.9 / 30.8.
+//   The always-on expert: beside the routed launches its passes compete for the chip, and the lines lie at 350 and 300 (4096 -> 1408, 48
+//   experts with one of 5632, Q8_0: 89 tokens 263 / 279, 113 tokens 272 / 329).
+//   Against coarse kernels alone, all four choices measured at 10935 random sizes (0.05 to 24 rows per expert): mean 0.813, 0.9 % are 3 % or
+//   more slower, 0.1 % by 10 %; with lines that count no empty workgroup 0.817, 2.1 % and 0.5 % (256 -> 512, 128 experts, top-1, Q4_0, layer, 640
+//   tokens 40.8 / 67.1).  Empty ones at a tenth, for a while, cost too much at sizes the fine kernels are made for (1024 -> 3584, eight experts,
+//   top-2, Q4_1, 65 tokens 60.5 / 37.7).
+inline bool q32_up_fine(int64_t F, const Q32Grid& g) {
+    const int64_t passes10 = 10 * g.live + 3 * (g.live - g.first), weight = g.kind == Q32Grid::LISTS ? 30 : 40;
+    return (F / 32 + 3) / 4 * passes10 / 10 + F / 32 * g.empty / weight <= (g.kind == Q32Grid::ALWAYS_ON ? 350 : 800);
 }
 inline bool q32_down_fine(int64_t H, const Q32Grid& g) {
-    const int64_t line = g.kind == Q32Grid::ROWS ? 400 : g.kind == Q32Grid::ALWAYS_ON ? 200 : 340;
-    return (H / 16 + 3) / 4 * g.live + H / 16 * g.empty / q32_empty_weight(g) <= line;
+    const int64_t weight = g.kind == Q32Grid::LISTS ? 30 : 20;
+    return (H / 16 + 3) / 4 * g.live + H / 16 * g.empty / weight <= (g.kind == Q32Grid::ALWAYS_ON ? 300 : 400);
 }
 
 }  // namespace moe

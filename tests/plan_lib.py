@@ -11,9 +11,9 @@ SOURCE = r"""
 #include "q32_plan.hpp"
 using namespace moe;
 // 1: fine up kernel, 2: fine down kernel
-extern "C" int fine(int64_t H, int64_t F, int64_t groups, int64_t k, int direct, int always_on, int tiles, int64_t T) {
+extern "C" int fine(int64_t H, int64_t F, int64_t groups, int64_t k, int direct, int always_on, int64_t T) {
     const Q32Grid g = q32_grid(T, k, groups, direct != 0, always_on != 0);
-    return q32_up_fine(F, g, tiles) + 2 * q32_down_fine(H, g);
+    return q32_up_fine(F, g) + 2 * q32_down_fine(H, g);
 }
 extern "C" int tiled32(int64_t T, int64_t k, int64_t E) { return q32_tiled(T, k, E); }
 // A tiled K-quant launch over `groups` lists: 1000 * tile + 10 * parts of K + (eight waves with rows of their own)
@@ -53,7 +53,7 @@ def load():
     lib = ctypes.CDLL(so)
     shutil.rmtree(d)
     i64, i = ctypes.c_int64, ctypes.c_int
-    lib.fine.argtypes = [i64, i64, i64, i64, i, i, i, i64]
+    lib.fine.argtypes = [i64, i64, i64, i64, i, i, i64]
     lib.tiled32.argtypes = [i64, i64, i64]
     lib.dense_kernel.argtypes = [i, i64, i64, i64]
     lib.up_kernel.argtypes = lib.down_kernel.argtypes = [i, i, i64, i64, i64, i64, i64]

@@ -12,23 +12,24 @@ def plan():
     return lib
 
 
-# (H, F, lists, top-k, direct, always on, slot tiles, tokens) -> 1: fine up projection, + 2: fine down projection.  us, coarse / fine
+# (H, F, lists, top-k, direct, always on, tokens) -> 1: fine up projection, + 2: fine down projection.  us, coarse / fine
 @pytest.mark.parametrize("args,want", [
-    ((1024, 3584, 8, 2, 1, 0, 1, 16), 3),       # 37.3 / 26.8
-    ((1024, 3584, 8, 2, 1, 0, 1, 40), 3),
-    ((1024, 3584, 8, 2, 1, 0, 1, 64), 2),       # lists of a second pass: up 20.8 / 22.6
-    ((4096, 14336, 8, 2, 1, 0, 1, 2), 3),       # up 85 / 56, 4 of 8 lists
-    ((4096, 14336, 8, 2, 1, 0, 1, 8), 0),       # 93 / 97
-    ((4096, 0, 1, 1, 0, 0, 1, 16), 3),          # dense products: 21.4 / 11.4
-    ((4096, 0, 1, 1, 0, 0, 4, 96), 3),          # 28.4 / 25.4
-    ((4096, 0, 1, 1, 0, 0, 4, 112), 1),         # 28.4 / 27.7, 512: 28.9 / 30.8
-    ((2048, 2816, 8, 4, 1, 0, 1, 28), 1),       # down, empty workgroups counted: layer 53.6 / 60.3
-    ((256, 512, 128, 1, 0, 0, 1, 400), 0),      # layer 35.7 / 52.2
-    ((256, 512, 128, 1, 0, 0, 1, 640), 0),      # 40.8 / 67.1
-    ((1024, 2816, 16, 1, 1, 0, 2, 260), 0),     # 60.9 / 96.1
-    ((4096, 5632, 1, 1, 0, 1, 4, 89), 0),       # always on, beside 48 experts: 263 / 279
-    ((4096, 5632, 1, 1, 0, 1, 4, 113), 0),      # 272 / 329
-    ((2048, 5632, 1, 1, 0, 1, 1, 16), 3),
+    ((1024, 3584, 8, 2, 1, 0, 16), 3),       # 37.3 / 26.8
+    ((1024, 3584, 8, 2, 1, 0, 40), 3),
+    ((1024, 3584, 8, 2, 1, 0, 65), 3),       # Q4_1, layer: 60.5 / 37.7
+    ((1024, 3584, 8, 2, 1, 0, 94), 3),       # 71 / 46
+    ((4096, 14336, 8, 2, 1, 0, 2), 3),       # up 85 / 56, 4 of 8 lists
+    ((4096, 14336, 8, 2, 1, 0, 3), 3),       # Q5_1, layer: 200 / 131
+    ((4096, 14336, 8, 2, 1, 0, 8), 0),       # 93 / 97
+    ((2048, 1408, 48, 4, 1, 0, 33), 1),      # Q5_0, four layers: 388 / 362
+    ((4096, 0, 1, 1, 0, 0, 16), 3),          # dense products: 21.4 / 11.4
+    ((4096, 0, 1, 1, 0, 0, 96), 3),          # 28.4 / 25.4
+    ((4096, 0, 1, 1, 0, 0, 112), 1),         # 28.4 / 27.7, 512: 28.9 / 30.8
+    ((256, 512, 128, 1, 0, 0, 400), 0),      # layer 35.7 / 52.2
+    ((256, 512, 128, 1, 0, 0, 640), 0),      # 40.8 / 67.1
+    ((1024, 2816, 16, 1, 1, 0, 260), 0),     # 60.9 / 96.1
+    ((4096, 5632, 1, 1, 0, 1, 113), 0),      # always on, beside 48 experts: 272 / 329
+    ((2048, 5632, 1, 1, 0, 1, 16), 3),
 ])
 def test_fine_kernels(plan, args, want):
     assert plan.fine(*args) == want
